@@ -505,7 +505,6 @@ extern "C" int qasr_hip_linear_bf16w(qasr_hip *h, float *y, const float *x, cons
     GemmArgs g{};
     g.M = (int)seq; g.N = (int)out_dim; g.K = (int)in_dim;
     g.A = x; g.lda = in_dim; g.B = w; g.ldb = in_dim; g.C = y; g.ldc = out_dim; g.bias = bias;
-    g.ws = reinterpret_cast<float *>(h->scratch); g.ws_bytes = QASR_SCRATCH_BYTES;   // split-K partials
     LAUNCHCHK(launch_gemm(g, A_F32_SPLIT, B_BF16, accumulate ? EPI_ACCUM : EPI_NONE, h->stream), "linear_bf16w");
     return QASR_OK;
 }
@@ -519,7 +518,6 @@ extern "C" int qasr_hip_gemm_w8_bf16(qasr_hip *h, float *y, const uint16_t *a, c
     GemmArgs g{};
     g.M = (int)M; g.N = (int)N; g.K = (int)K;
     g.A = a; g.lda = K; g.B = w; g.ldb = K; g.C = y; g.ldc = N; g.scale = scales;
-    g.ws = reinterpret_cast<float *>(h->scratch); g.ws_bytes = QASR_SCRATCH_BYTES;   // split-K partials
     LAUNCHCHK(launch_gemm(g, A_BF16, B_I8, EPI_SCALE, h->stream), "gemm_w8_bf16");
     return QASR_OK;
 }

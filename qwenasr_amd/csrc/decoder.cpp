@@ -198,8 +198,9 @@ int decoder_build(qasr_decoder *d, const qasr_dec_weights *w, const uint16_t *lm
     const int64_t kvd = (int64_t)c.n_kv_heads * hd, I = c.intermediate, V = c.vocab;
     const int64_t nqkv = qd + 2 * kvd;
     // every matrix goes host -> HBM through the pinned staging ring (the q|k|v
-    // concatenation and the gate/up interleave are assembled on the way) and
-    // is packed to int8 on the device behind its upload
+    // concatenation and the gate/up interleave are assembled on the way), is
+    // packed to int8 on the device behind its upload and then laid out
+    // fragment-major for the prefill GEMMs
     Stager stg(d->h->stream);
     TRY(stg.init());
     const size_t B2 = sizeof(uint16_t);
@@ -213,17 +214,21 @@ int decoder_build(qasr_decoder *d, const qasr_dec_weights *w, const uint16_t *lm
         TRY(stg.upload(D.bqkv + qd * H, S.wk, B2 * kvd * H));
         TRY(stg.upload(D.bqkv + (qd + kvd) * H, S.wv, B2 * kvd * H));
         TRY(pack(d, D.bqkv, nqkv, H, &D.wqkv, &D.sqkv));
+        LAUNCHCHK(launch_pack_frag(D.bqkv, nqkv, H, d->h->stream), "weight layout");
         TRY(dalloc(d, &D.bo, H * qd));
         TRY(stg.upload(D.bo, S.wo, B2 * H * qd));
         TRY(pack(d, D.bo, H, qd, &D.wo, &D.so));
+        LAUNCHCHK(launch_pack_frag(D.bo, H, qd, d->h->stream), "weight layout");
         // gate/up interleaved by rows (decoder.rs:91-104)
         TRY(dalloc(d, &D.bgu, 2 * I * H));
         const void *gu[2] = {S.gate, S.up};
         TRY(stg.upload_rows(D.bgu, gu, 2, I, B2 * H));
         TRY(pack(d, D.bgu, 2 * I, H, &D.wgu, &D.sgu));
+        LAUNCHCHK(launch_pack_frag(D.bgu, 2 * I, H, d->h->stream), "weight layout");
         TRY(dalloc(d, &D.bdown, H * I));
         TRY(stg.upload(D.bdown, S.down, B2 * H * I));
         TRY(pack(d, D.bdown, H, I, &D.wdown, &D.sdown));
+        LAUNCHCHK(launch_pack_frag(D.bdown, H, I, d->h->stream), "weight layout");
         TRY(dalloc(d, &D.q_norm, hd));
         TRY(dalloc(d, &D.k_norm, hd));
         TRY(dalloc(d, &D.in_norm, H));
@@ -285,7 +290,6 @@ extern "C" void qasr_hip_decoder_free(qasr_decoder *d) {
     for (auto &g : d->graphs) (void)hipGraphExecDestroy(g.second);
     decoder_free_prefill(d);
     dbuf_release(d->head_out);
-    dbuf_release(d->gemm_ws);
     if (d->lm_bf16) (void)hipFree(d->lm_bf16);
     for (void *p : d->allocs) (void)hipFree(p);
     delete d;

@@ -55,7 +55,6 @@ struct qasr_decoder {
     int32_t host_state[4] = {0, 0, 0, 0};
     PrefillBufs pf;
     DevBuf head_out;                            // prefill_logits / prefill_argmax outputs, kept between calls
-    DevBuf gemm_ws;                             // the prefill GEMMs' split-K partials (2 x rows x 1024 f32)
     std::vector<void *> allocs;
 };
 

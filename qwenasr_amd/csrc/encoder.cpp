@@ -120,6 +120,19 @@ static int eupload_big(qasr_encoder *e, Stager &stg, T **p, const T *host, size_
     return stg.upload(*p, host, count * sizeof(T));
 }
 
+// A layer's matrix: uploaded as rows, then fragment-major where the GEMM takes
+// that (K % 32 == 0).  The layouts run together after the last upload: one
+// between every two copies makes the copy engine and the compute queue wait
+// for each other (the encoder's load 14.4 -> 16.0 ms).
+struct EncMat { uint16_t *w; int64_t N, K; };
+
+static int eupload_mat(qasr_encoder *e, Stager &stg, std::vector<EncMat> &mats, uint16_t **p, const uint16_t *host,
+                       int64_t N, int64_t K) {
+    TRY(ealloc(e, p, (size_t)(gemm_frag_rows(N) * K)));
+    mats.push_back({*p, N, K});
+    return stg.upload(*p, host, sizeof(uint16_t) * N * K);
+}
+
 static int encoder_build(qasr_encoder *e, const qasr_enc_weights *w) {
     const qasr_enc_config &c = e->c;
     const int64_t D = c.d_model, F = c.ffn_dim, C = c.conv_hidden, O = c.output_dim;
@@ -130,7 +143,7 @@ static int encoder_build(qasr_encoder *e, const qasr_enc_weights *w) {
     e->stem_nhwc = C % 32 == 0;
     if (e->stem_nhwc) {
         // each matrix staged as the reference holds it ([out][channel][tap]),
-        // then reordered on the device to [out][tap][channel]; the staging
+        // then reordered on the device to fragment-major (tap, channel); the staging
         // buffer is reused in stream order and freed once the stream drains
         uint16_t *raw = nullptr;
         const size_t raw_n = (size_t)std::max(C * C * 9, D * C * h3);
@@ -140,7 +153,7 @@ static int encoder_build(qasr_encoder *e, const qasr_enc_weights *w) {
             {&e->conv2_w, w->conv2_w, C, 9}, {&e->conv3_w, w->conv3_w, C, 9}, {&e->conv_out_w, w->conv_out_w, D, h3}};
         int rc = QASR_OK;
         for (const auto &m : mats) {
-            if (rc == QASR_OK) rc = ealloc(e, m.dst, (size_t)(m.o * C * m.t));
+            if (rc == QASR_OK) rc = ealloc(e, m.dst, (size_t)(gemm_frag_rows(m.o) * C * m.t));
             if (rc == QASR_OK) rc = stg.upload(raw, m.src, sizeof(uint16_t) * m.o * C * m.t);
             if (rc == QASR_OK && launch_taps_last(*m.dst, raw, (int)m.o, (int)C, (int)m.t, e->h->stream) != hipSuccess)
                 rc = qasr_fail(QASR_ERR_HIP, "encoder: weight reorder failed");
@@ -159,22 +172,24 @@ static int encoder_build(qasr_encoder *e, const qasr_enc_weights *w) {
     TRY(eupload(e, &e->conv2_b, w->conv2_b, C));
     TRY(eupload(e, &e->conv3_b, w->conv3_b, C));
     e->L.resize(c.n_layers);
+    std::vector<EncMat> mats;
     for (int l = 0; l < c.n_layers; l++) {
         const qasr_enc_layer &s = w->layers[l];
         EncLayerDev &L = e->L[l];
-        TRY(ealloc(e, &L.wqkv, 3 * D * D));
+        TRY(ealloc(e, &L.wqkv, gemm_frag_rows(3 * D) * D));
         TRY(stg.upload(L.wqkv, s.wq, 2 * D * D));
         TRY(stg.upload(L.wqkv + D * D, s.wk, 2 * D * D));
         TRY(stg.upload(L.wqkv + 2 * D * D, s.wv, 2 * D * D));
+        mats.push_back({L.wqkv, 3 * D, D});
         TRY(ealloc(e, &L.bqkv, 3 * D));
         HIPCHK(hipMemcpyAsync(L.bqkv, s.bq, D * 4, hipMemcpyHostToDevice, e->h->stream));
         HIPCHK(hipMemcpyAsync(L.bqkv + D, s.bk, D * 4, hipMemcpyHostToDevice, e->h->stream));
         HIPCHK(hipMemcpyAsync(L.bqkv + 2 * D, s.bv, D * 4, hipMemcpyHostToDevice, e->h->stream));
-        TRY(eupload_big(e, stg, &L.wo, s.wo, D * D));
+        TRY(eupload_mat(e, stg, mats, &L.wo, s.wo, D, D));
         TRY(eupload(e, &L.bo, s.bo, D));
-        TRY(eupload_big(e, stg, &L.fc1, s.fc1, F * D));
+        TRY(eupload_mat(e, stg, mats, &L.fc1, s.fc1, F, D));
         TRY(eupload(e, &L.b1, s.b1, F));
-        TRY(eupload_big(e, stg, &L.fc2, s.fc2, D * F));
+        TRY(eupload_mat(e, stg, mats, &L.fc2, s.fc2, D, F));
         TRY(eupload(e, &L.b2, s.b2, D));
         TRY(eupload(e, &L.ln1_w, s.ln1_w, D));
         TRY(eupload(e, &L.ln1_b, s.ln1_b, D));
@@ -183,10 +198,12 @@ static int encoder_build(qasr_encoder *e, const qasr_enc_weights *w) {
     }
     TRY(eupload(e, &e->ln_post_w, w->ln_post_w, D));
     TRY(eupload(e, &e->ln_post_b, w->ln_post_b, D));
-    TRY(eupload_big(e, stg, &e->proj1_w, w->proj1_w, D * D));
+    TRY(eupload_mat(e, stg, mats, &e->proj1_w, w->proj1_w, D, D));
     TRY(eupload(e, &e->proj1_b, w->proj1_b, D));
-    TRY(eupload_big(e, stg, &e->proj2_w, w->proj2_w, O * D));
+    TRY(eupload_mat(e, stg, mats, &e->proj2_w, w->proj2_w, O, D));
     TRY(eupload(e, &e->proj2_b, w->proj2_b, O));
+    for (const EncMat &m : mats)
+        if (gemm_frag_ok(m.K)) LAUNCHCHK(launch_pack_frag(m.w, m.N, m.K, e->h->stream), "encoder weight layout");
     // per-chunk sinusoidal PE (sinusoidal_pe, kernels/mod.rs:1704-1717)
     e->tokens_per_chunk = conv_len(conv_len(conv_len(c.chunk_size)));
     {
@@ -270,17 +287,21 @@ int64_t encoder_tokens(const qasr_encoder *e, int64_t frames) {
 
 static int egemm(qasr_encoder *e, const float *A, int64_t lda, const uint16_t *B, int64_t ldb, float *C,
                  int64_t ldc, int M, int N, int K, const float *bias, int epi, int64_t gelu_n = 0,
-                 int gelu_rows = 0) {
+                 int gelu_rows = 0, int bsrc = B_BF16) {
     GemmArgs g{};
     g.M = M; g.N = N; g.K = K;
     g.A = A; g.lda = lda; g.B = B; g.ldb = ldb; g.C = C; g.ldc = ldc; g.bias = bias;
     g.gelu_n = gelu_n; g.gelu_rows = gelu_rows;
-    g.ws = reinterpret_cast<float *>(e->h->scratch); g.ws_bytes = QASR_SCRATCH_BYTES;
-    // K split chosen by the shape alone: a row's bits do not depend on how many
-    // rows (sequences) share the call
-    g.split_by_shape = 1;
-    LAUNCHCHK(launch_gemm(g, A_F32_SPLIT, B_BF16, epi, e->h->stream), "encoder gemm");
+    // (K slices go with the shape alone: a row's bits do not depend on how many
+    // rows, or sequences, share the call)
+    LAUNCHCHK(launch_gemm(g, A_F32_SPLIT, bsrc, epi, e->h->stream), "encoder gemm");
     return QASR_OK;
+}
+
+// egemm on one of the layers' matrices (eupload_mat's layout)
+static int emat(qasr_encoder *e, const float *A, int64_t lda, const uint16_t *B, int64_t ldb, float *C, int64_t ldc,
+                int M, int N, int K, const float *bias, int epi, int64_t gelu_n = 0) {
+    return egemm(e, A, lda, B, ldb, C, ldc, M, N, K, bias, epi, gelu_n, 0, gemm_frag_ok(K) ? B_BF16_FRAG : B_BF16);
 }
 
 // implicit-im2col GEMM of a channels-last convolution (K in (tap, channel)
@@ -294,7 +315,7 @@ static int econv(qasr_encoder *e, const float *in, int n_chunks, int hin, int wi
     g.gelu_n = (int64_t)N * hout * wout; g.gelu_rows = hout * wout;
     g.conv_hin = hin; g.conv_win = win; g.conv_c = cin; g.conv_hout = hout; g.conv_wout = wout;
     g.conv_kh = kh; g.conv_kw = kw; g.conv_sy = sy; g.conv_sx = sx; g.conv_py = py; g.conv_px = px;
-    LAUNCHCHK(launch_gemm(g, A_CONV, B_BF16, epi, e->h->stream), "encoder conv gemm");
+    LAUNCHCHK(launch_gemm(g, A_CONV, B_BF16_FRAG, epi, e->h->stream), "encoder conv gemm");
     return QASR_OK;
 }
 
@@ -443,7 +464,7 @@ int encoder_forward_multi(qasr_encoder *e, int n, const float *const *mels, cons
     for (int l = 0; l < c.n_layers; l++) {
         const EncLayerDev &L = e->L[l];
         LAUNCHCHK(launch_layer_norm_rows(xn, x, L.ln1_w, L.ln1_b, Mt, D, 1e-5f, st), "enc ln1");
-        TRY(egemm(e, xn, D, L.wqkv, D, qkv, 3 * D, M, 3 * D, D, L.bqkv, EPI_NONE));
+        TRY(emat(e, xn, D, L.wqkv, D, qkv, 3 * D, M, 3 * D, D, L.bqkv, EPI_NONE));
         AttnRowsArgs a{};
         a.q = qkv; a.q_rs = 3 * D;
         a.k = qkv + D; a.v = qkv + 2 * D; a.k_hs = c.head_dim; a.k_rs = 3 * D;
@@ -458,16 +479,16 @@ int encoder_forward_multi(qasr_encoder *e, int n, const float *const *mels, cons
             }
         }
         LAUNCHCHK(launch_attn_rows(a, c.n_heads, c.head_dim, st), "enc attention");
-        TRY(egemm(e, att, D, L.wo, D, x, D, M, D, D, L.bo, EPI_ACCUM));
+        TRY(emat(e, att, D, L.wo, D, x, D, M, D, D, L.bo, EPI_ACCUM));
         LAUNCHCHK(launch_layer_norm_rows(xn, x, L.ln2_w, L.ln2_b, Mt, D, 1e-5f, st), "enc ln2");
-        TRY(egemm(e, xn, D, L.fc1, D, mid, F, M, F, D, L.b1, EPI_GELU, (int64_t)Mt * F));
-        TRY(egemm(e, mid, F, L.fc2, F, x, D, M, D, F, L.b2, EPI_ACCUM));
+        TRY(emat(e, xn, D, L.fc1, D, mid, F, M, F, D, L.b1, EPI_GELU, (int64_t)Mt * F));
+        TRY(emat(e, mid, F, L.fc2, F, x, D, M, D, F, L.b2, EPI_ACCUM));
     }
     LAUNCHCHK(launch_layer_norm_rows(xn, x, e->ln_post_w, e->ln_post_b, Mt, D, 1e-5f, st), "enc ln_post");
-    TRY(egemm(e, xn, D, e->proj1_w, D, att, D, M, D, D, e->proj1_b, EPI_GELU, (int64_t)Mt * D));
+    TRY(emat(e, xn, D, e->proj1_w, D, att, D, M, D, D, e->proj1_b, EPI_GELU, (int64_t)Mt * D));
     int64_t off = 0;
     for (int j = 0; j < n; j++) {
-        TRY(egemm(e, att + P[j] * D, D, e->proj2_w, D, out + off * O, O, (int)T[j], O, D, e->proj2_b, EPI_NONE));
+        TRY(emat(e, att + P[j] * D, D, e->proj2_w, D, out + off * O, O, (int)T[j], O, D, e->proj2_b, EPI_NONE));
         tokens[j] = T[j];
         off += T[j];
     }

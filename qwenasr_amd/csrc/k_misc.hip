@@ -350,24 +350,25 @@ hipError_t launch_conv1_direct(float *out, const float *in, int n_chunks, int64_
     return hipGetLastError();
 }
 
-// w[o][c][t] -> out[o][t][c] (bf16): a convolution's weights with the K index
-// (channel, tap) reordered to (tap, channel), the order of the channels-last
-// implicit-im2col GEMM
+// w[o][c][t] (bf16) -> the fragment-major weights (launch_pack_frag's layout) of
+// the channels-last implicit-im2col GEMM, whose K index is (tap, channel);
+// rows past O (a last partial group of 16) are zeros.  Cin % 32 == 0.
 __global__ __launch_bounds__(256) void k_taps_last(uint16_t *__restrict__ out, const uint16_t *__restrict__ in,
                                                    int O, int Cin, int T) {
-    const int64_t total = (int64_t)O * Cin * T;
+    const int nk = Cin / 32 * T;
+    const int64_t total = (int64_t)((O + 15) / 16) * nk * 512;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-        const int c = (int)(i % Cin);
-        const int64_t r = i / Cin;
-        const int t = (int)(r % T);
-        const int64_t o = r / T;
-        out[i] = in[(o * Cin + c) * T + t];
+        const int e = (int)(i & 511), l = e >> 3;
+        const int64_t f = i >> 9;
+        const int o = (int)(f / nk) * 16 + (l & 15), k = (int)(f % nk) * 32 + (l >> 4) * 8 + (e & 7);
+        const int t = k / Cin, c = k - t * Cin;
+        out[i] = o < O ? in[((int64_t)o * Cin + c) * T + t] : (uint16_t)0;
     }
 }
 
 hipError_t launch_taps_last(uint16_t *out, const uint16_t *in, int O, int Cin, int T, hipStream_t st) {
-    if (O <= 0 || Cin <= 0 || T <= 0) return hipErrorInvalidValue;
-    const int64_t total = (int64_t)O * Cin * T;
+    if (O <= 0 || Cin <= 0 || Cin % 32 != 0 || T <= 0) return hipErrorInvalidValue;
+    const int64_t total = (int64_t)gemm_frag_rows(O) * Cin * T;
     const unsigned blocks = (unsigned)std::min<int64_t>((total + 255) / 256, 65536);
     hipLaunchKernelGGL(k_taps_last, dim3(blocks), dim3(256), 0, st, out, in, O, Cin, T);
     return hipGetLastError();

@@ -197,7 +197,8 @@ hipError_t launch_head_norm_rope(float *x, const float *w, const float *cos_t, c
 namespace qasr {
 // ---- GEMM ----------------------------------------------------------------
 enum { A_F32_SPLIT = 0, A_BF16 = 1, A_CONV = 2 };
-enum { B_BF16 = 0, B_I8 = 1 };
+// B_BF16_FRAG: the bf16 weights fragment-major (launch_pack_frag)
+enum { B_BF16 = 0, B_I8 = 1, B_BF16_FRAG = 2 };
 // EPI_SWIGLU: B rows interleave (gate, up); C[m][n / 2] = silu(gate) up (ldc
 // in outputs, N / 2 of them), the decoder's SwiGLU with its AVX / tail paths
 enum { EPI_NONE = 0, EPI_ACCUM = 1, EPI_SCALE = 2, EPI_GELU = 4, EPI_TRANS = 8, EPI_CHW = 16, EPI_SWIGLU = 32 };
@@ -215,12 +216,6 @@ struct GemmArgs {
     int64_t gelu_n;           // elements of the buffer gelu() sees (EPI_GELU / EPI_TRANS: per chunk)
     int gelu_rows;            // EPI_TRANS: spatial positions per chunk
     int a_vec4, b_vec;        // set by the launcher
-    float *ws;                // optional workspace for split-K partials (null: no split)
-    int64_t ws_bytes;
-    // f32-class path: split K by the shape alone (N <= 1024 and K / 32 >= 16),
-    // whatever M, so that a row's result does not depend on how many rows
-    // share the call; the launch fails if the workspace is too small
-    int split_by_shape;
     // A_CONV (f32-class, implicit im2col): A is a channels-last activation
     // [chunks][conv_hin][conv_win][conv_c]; GEMM row m is output position
     // (chunk, oy, ox) of a conv_hout x conv_wout grid and K index (ky, kx, c)
@@ -228,9 +223,19 @@ struct GemmArgs {
     // zero outside the input.  conv_c % 32 == 0.
     int conv_hin, conv_win, conv_c, conv_hout, conv_wout, conv_kh, conv_kw, conv_sy, conv_sx, conv_py, conv_px;
     float conv_rc, conv_rkw;  // 1 / conv_c, 1 / conv_kw (set by the launcher)
+    int m_major;              // tile order of k_gemm_ks (set by the launcher)
 };
 
 hipError_t launch_gemm(const GemmArgs &g, int asrc, int bsrc, int epi, hipStream_t st);
+// the f32-class kernel behind launch_gemm (k_gemm_ks.hip) and what it takes
+bool gemm_ks_ok(const GemmArgs &g, int asrc, int bsrc, int epi);
+hipError_t launch_gemm_ks(const GemmArgs &g, int asrc, int bsrc, int epi, hipStream_t st);
+// B [N][K] bf16 rows -> fragment-major in place, for K that gemm_frag_ok
+// allows; the buffer holds gemm_frag_rows(N) rows
+#define GEMM_FRAG_MAX_K 8192
+inline bool gemm_frag_ok(int64_t K) { return K > 0 && K % 32 == 0 && K <= GEMM_FRAG_MAX_K; }
+inline int64_t gemm_frag_rows(int64_t N) { return (N + 15) / 16 * 16; }
+hipError_t launch_pack_frag(uint16_t *b, int64_t N, int64_t K, hipStream_t st);
 hipError_t launch_gemm_f32(const GemmArgs &g, hipStream_t st);
 }  // namespace qasr
 

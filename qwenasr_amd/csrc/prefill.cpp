@@ -38,17 +38,15 @@ static int ensure_prefill(qasr_decoder *d, int64_t S) {
     return QASR_OK;
 }
 
-// The prefill GEMMs split K by the shape alone (split_by_shape), so that a
-// row's result is the same whether its sequence is prefilled alone or with
-// others; their partials live in the decoder's grow-only workspace.
+// The f32-class GEMMs slice K by the shape alone, so that a row's result is the
+// same whether its sequence is prefilled alone or with others.  The layers'
+// weights and a separate head are fragment-major, the tied embedding is rows.
 static int gemm(qasr_decoder *d, const float *A, int64_t lda, const uint16_t *B, int64_t ldb, float *C,
-                int64_t ldc, int M, int N, int K, int epi) {
+                int64_t ldc, int M, int N, int K, int epi, int bsrc = B_BF16_FRAG) {
     GemmArgs g{};
     g.M = M; g.N = N; g.K = K;
     g.A = A; g.lda = lda; g.B = B; g.ldb = ldb; g.C = C; g.ldc = ldc;
-    g.ws = d->gemm_ws.as<float>(); g.ws_bytes = (int64_t)d->gemm_ws.cap;   // split-K partials
-    g.split_by_shape = 1;
-    LAUNCHCHK(launch_gemm(g, A_F32_SPLIT, B_BF16, epi, d->h->stream), "prefill gemm");
+    LAUNCHCHK(launch_gemm(g, A_F32_SPLIT, bsrc, epi, d->h->stream), "prefill gemm");
     return QASR_OK;
 }
 
@@ -74,7 +72,6 @@ int decoder_prefill_segments(qasr_decoder *d, const PrefillSeg *segs, int n_seg)
     if (S <= 0) return QASR_OK;
     if (S > (1 << 30) / 8) return qasr_fail(QASR_ERR_INVALID, "decoder_prefill: too many rows");
     TRY(ensure_prefill(d, S));
-    TRY(dbuf_ensure(d->gemm_ws, sizeof(float) * 2 * (size_t)S * 1024, d->h->stream));
     hipStream_t st = d->h->stream;
     PrefillBufs &p = d->pf;
     const int H = c.hidden, hd = c.head_dim, qd = c.n_heads * hd, kvd = c.n_kv_heads * hd;
@@ -228,7 +225,7 @@ extern "C" int qasr_hip_decoder_set_lm_head(qasr_decoder *d, const uint16_t *w, 
     if (!w) return QASR_OK;
     if (out_dim <= 0) return qasr_fail(QASR_ERR_INVALID, "set_lm_head: out_dim must be positive");
     const size_t bytes = sizeof(uint16_t) * out_dim * d->c.hidden;
-    if (hipMalloc(&d->lm_bf16, bytes) != hipSuccess) {
+    if (hipMalloc(&d->lm_bf16, sizeof(uint16_t) * gemm_frag_rows(out_dim) * d->c.hidden) != hipSuccess) {
         d->lm_bf16 = nullptr;
         return qasr_fail(QASR_ERR_NOMEM, "set_lm_head: device allocation failed");
     }
@@ -238,6 +235,11 @@ extern "C" int qasr_hip_decoder_set_lm_head(qasr_decoder *d, const uint16_t *w, 
         (void)hipFree(d->lm_bf16);
         d->lm_bf16 = nullptr;
         return qasr_fail(QASR_ERR_HIP, "set_lm_head: upload failed");
+    }
+    if (launch_pack_frag(d->lm_bf16, out_dim, d->c.hidden, d->h->stream) != hipSuccess) {
+        (void)hipFree(d->lm_bf16);
+        d->lm_bf16 = nullptr;
+        return qasr_fail(QASR_ERR_HIP, "set_lm_head: layout failed");
     }
     d->lm_rows = out_dim;
     return QASR_OK;
@@ -289,7 +291,8 @@ static int prefill_head_rows(qasr_decoder *d, const float *embeds, int64_t seq_l
             src = d->pf.gu;
         }
         LAUNCHCHK(launch_rms_norm_rows(d->pf.xn, src, d->norm, n, (int)H, d->c.eps, st), "logits rms_norm");
-        TRY(gemm(d, d->pf.xn, H, w, H, y, out_dim, (int)n, (int)out_dim, (int)H, EPI_NONE));
+        TRY(gemm(d, d->pf.xn, H, w, H, y, out_dim, (int)n, (int)out_dim, (int)H, EPI_NONE,
+                 d->lm_bf16 ? B_BF16_FRAG : B_BF16));
         if (logits)
             HIPCHK(hipMemcpyAsync(logits, y, sizeof(float) * n * out_dim, hipMemcpyDeviceToHost, st));
         if (idx) {

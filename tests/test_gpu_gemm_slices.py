@@ -1,0 +1,60 @@
+"""The K-sliced f32-class GEMM at the edges of its tile forms.
+
+Plain-row weights through the `linear` operator and fragment-major weights
+through `prefill_logits` with a separate head; the two layouts run the same
+sums, so their results are compared bit for bit.
+"""
+import numpy as np
+import pytest
+
+from conftest import bf16, bf16f, rng
+
+pytestmark = pytest.mark.gpu
+
+# 8 K slices below 2048 columns, 4 from there on; fewer K-steps than slices;
+# partial row and column tiles of every form (16 x 32 ... 32 x 128, 64 x 64)
+SHAPES = [(1, 64, 32), (16, 1023, 512), (33, 2047, 96), (129, 1000, 2048), (600, 96, 1024), (2100, 1030, 64),
+          (15, 2048, 32), (40, 2050, 160), (300, 2303, 1024), (1500, 2049, 64), (700, 6150, 96)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_linear_slices(dev, M, N, K):
+    from qwenasr_amd import kernels as Kr
+    print(f"linear slices M={M} N={N} K={K}", flush=True)
+    r = rng(M * 7 + N * 3 + K)
+    x = r.normal(0, 1, (M, K)).astype(np.float32)
+    w = bf16(r.normal(0, 0.02, (N, K)))
+    dx, dw = dev.upload(x), dev.upload(w)
+    y = dev.zeros((M + 1, N), np.float32)
+    Kr.linear(y, dx, dw, None, M, K, N)
+    got = y.numpy()
+    xd, wd = x.astype(np.float64), bf16f(w).astype(np.float64)
+    exact = xd @ wd.T
+    # K roundings of partial sums no larger than sum |x w|, each at most 2^-24
+    bound = K * 2.0 ** -24 * (np.abs(xd) @ np.abs(wd).T) + 1e-30
+    assert (np.abs(got[:M] - exact) <= bound).all()
+    assert (got[M] == 0).all()                       # nothing past the last row
+    # a row's bits do not depend on how many rows share the call
+    y1 = dev.empty((1, N), np.float32)
+    Kr.linear(y1, dev.upload(x[M - 1:]), dw, None, 1, K, N)
+    assert (y1.numpy()[0] == got[M - 1]).all()
+
+
+@pytest.mark.parametrize("hidden,inter,vocab,rows", [(64, 64, 33, 1), (192, 320, 1003, 17), (1024, 448, 2050, 70),
+                                                     (256, 192, 2047, 300)])
+def test_fragment_major_head(dev, hidden, inter, vocab, rows):
+    """A separate head equal to the tied embedding (plain rows) gives its bits."""
+    from qwenasr_amd.model import Decoder
+    from qwenasr_amd.synth import SynthDecoder
+    print(f"head layouts hidden={hidden} vocab={vocab} rows={rows}", flush=True)
+    cfg = dict(n_layers=1, hidden=hidden, n_heads=16, n_kv_heads=8, head_dim=128, intermediate=inter, vocab=vocab,
+               eps=1e-6, theta=1e6)
+    w = SynthDecoder(cfg, seed=77)
+    d = Decoder(dev, w, max_seq=512)
+    emb = rng(rows).normal(0, 0.05, (rows, hidden)).astype(np.float32)
+    tied = d.prefill_logits(emb)
+    d.kv_len = 0
+    d.set_lm_head(w.embed)
+    own = d.prefill_logits(emb)
+    d.close()
+    assert np.isfinite(tied).all() and (tied == own).all()
