@@ -4,6 +4,7 @@
 #include <cstdlib>
 
 #include "kernels.h"
+#include "gemm_common.h"
 
 namespace qasr {
 
@@ -630,38 +631,44 @@ __global__ __launch_bounds__(256) void k_attn_rows(AttnRowsArgs a) {
 
 // ---------------------------------------------------------------------------
 // The same multi-row attention on f32 MFMA (v_mfma_f32_16x16x4_f32, exact f32
-// products, f32 accumulation).  A block owns 16 query rows of the G query
-// heads of one KV head; its NW waves are (head g, key split ks), G x KS = NW,
-// and wave (g, ks) takes the 16-key sub-tiles ks, ks + KS, ... of every
-// KS x 16-key chunk staged in LDS, with an online softmax of its own; the KS
-// states of a head are merged through LDS at the end.  The next chunk's K/V
-// loads go out into registers before the current chunk's MFMA work.  With
-// kv_div = 2 (and G = 1) a block owns one query head x and reads KV head x / 2,
-// which gives the 8 waves of a 128-dim head 8 key splits.  Per sub-tile the wave
-// forms S^T = K Q^T (16 keys x 16 queries; lane l holds keys 4 (l / 16) + i
-// of query l % 16, the dot over d split as lane group l / 16 covering dims
-// [l/16 HD/4, +HD/4)), so the softmax of a query reduces over the lane's 4
-// values and two cross-group shuffles, and the probabilities already sit in
-// the A-operand layout of O += P V (query l % 16, key 4 (l / 16) + i at step
-// i).  The O rows a lane accumulates are queries 4 (l / 16) + j, whose
-// rescale factors come from the lanes owning those queries.
+// products, f32 accumulation).  A block owns 16 query rows of one query head
+// (KV head blockIdx.x / kv_div); its NW waves split the keys: wave w takes the
+// 16-key sub-tiles w, w + NW, ... with an online softmax of its own, and the NW
+// states are merged through LDS at the end.
+//
+// Every wave streams its sub-tiles alone through an LDS stage of its own: K by
+// global_load_lds, refilled as soon as its fragments are in registers, and V
+// the same way, so that the next K rows travel during this sub-tile's softmax
+// and P V and the next V rows during the next scores; no barrier before the
+// merge.  (Before, the block staged 128-key chunks through registers: load,
+// LDS store, barrier, compute in turn, the matrix cores idle for half of each
+// chunk.)  What bounds it: 64 MFMAs of 32 clk per sub-tile, 145 TFLOP/s over
+// the chip at best, and for short prompts the longest block's chain.
+//
+// Per sub-tile the wave forms S^T = K Q^T (16 keys x 16 queries; lane l holds
+// keys 4 (l / 16) + i of query l % 16, the dot over d split as lane group l /
+// 16 covering dims [l/16 HD/4, +HD/4)), so the softmax of a query reduces over
+// the lane's 4 values and two cross-group shuffles, and the probabilities
+// already sit in the A-operand layout of O += P V (query l % 16, key 4 (l / 16)
+// + i at step i).  Column l % 16 of the B operand's tile n is dim NT (l % 16)
+// + n: a lane reads its NT values of a V row as whole 16-byte slots.  The O
+// rows a lane accumulates are queries 4 (l / 16) + j, whose rescale factors
+// come from the lanes owning those queries.
+//
+// LDS placement: slot q (16 bytes) of K row r sits at q ^ (r & 7): the 16 rows
+// of a fragment read fall in different banks; V rows are read along the row.
 // ---------------------------------------------------------------------------
-// One block's work: query rows [q0, q0 + 16) of the KV head (pair) blockIdx.x.
-template <int HD, int G, int NW>
+// One block's work: query rows [q0, q0 + 16) of query head blockIdx.x.
+template <int HD, int NW>
 __device__ __forceinline__ void attn_mfma_block(const AttnRowsArgs &a, int q0) {
-    constexpr int KS = NW / G, CH = 16 * KS, NST = HD / 4, NT = HD / 16, LD = HD + 4;
-    constexpr int NTH = NW * 64, SV = CH * (HD / 4) / NTH;   // float4 of K (and of V) staged per thread
-    static_assert(CH * (HD / 4) % NTH == 0, "staging");
-    // one LDS buffer: K and V chunks [CH][LD] during the loop, the waves' O rows after it
-    static_assert(2 * CH * LD >= NW * 16 * HD, "merge buffer");
-    __shared__ __attribute__((aligned(16))) float smem[2 * CH * LD];
-    float (*Ks)[LD] = reinterpret_cast<float (*)[LD]>(smem);
-    float (*Vs)[LD] = reinterpret_cast<float (*)[LD]>(smem + CH * LD);
+    constexpr int NST = HD / 4, NT = HD / 16;
+    constexpr int RB = HD * 4, TB = 16 * RB;               // bytes of a K or V row, of a 16-key tile
+    constexpr int LPR = RB / 16, RPL = 64 / LPR, L = 16 / RPL;   // lanes per row, rows per load, loads per tile
+    __shared__ __attribute__((aligned(16))) char smem[NW * 2 * TB];
+    __shared__ float Mm[NW][16], Ll[NW][16], Ff[NW][16];
     const int t = threadIdx.x, lane = t & 63;
     const int wid = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int g = wid / KS, ks = wid % KS;
-    const int kvh = blockIdx.x;
-    const int h = kvh * G + g;
+    const int h = blockIdx.x;
     const int lq = lane & 15, lg = lane >> 4;
     // key range of this lane's query (for the S^T masks) and of the block
     const int qi = q0 + lq;
@@ -687,6 +694,25 @@ __device__ __forceinline__ void attn_mfma_block(const AttnRowsArgs &a, int q0) {
         blo = 0;
         bhi = min(a.q_offset + qlast + 1, a.n_k);
     }
+    const int kv_head = a.kv_div > 1 ? h / a.kv_div : h;
+    const float *kb = a.k + (int64_t)kv_head * a.k_hs, *vb = a.v + (int64_t)kv_head * a.k_hs;
+    char *Ks = smem + wid * 2 * TB, *Vs = Ks + TB;
+    // tile c (keys blo + 16 c ...): rows past the range repeat its last one (their scores are masked)
+    const int n_sub = (bhi - blo + 15) / 16, lr = lane / LPR, ls = lane % LPR;
+    auto issue = [&](const float *base, char *dst, int c, bool swz) {
+        const int j0 = blo + 16 * c, last = bhi - 1 - j0;
+        const char *p = reinterpret_cast<const char *>(base + (int64_t)j0 * a.k_rs);
+#pragma unroll
+        for (int u = 0; u < L; u++) {
+            const int r = u * RPL + lr;
+            const uint32_t off = (uint32_t)min(r, last) * (uint32_t)a.k_rs * 4u + 16 * (swz ? ls ^ (r & 7) : ls);
+            lds_dma16_s(p, off, dst + 1024 * u);
+        }
+    };
+    if (wid < n_sub) {
+        issue(kb, Ks, wid, true);
+        issue(vb, Vs, wid, false);
+    }
     // this lane's slice of q: dims [lg NST, lg NST + NST) of query qi, head h
     float qv[NST];
     {
@@ -697,63 +723,40 @@ __device__ __forceinline__ void attn_mfma_block(const AttnRowsArgs &a, int q0) {
             qv[s] = x.x; qv[s + 1] = x.y; qv[s + 2] = x.z; qv[s + 3] = x.w;
         }
     }
+#pragma unroll
+    for (int s = 0; s < NST; s++) asm volatile("" : "+v"(qv[s]));   // waited for here, not inside the loop
     f32x4 o[NT];
 #pragma unroll
     for (int n = 0; n < NT; n++) o[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     float m = -INFINITY, l = 0.0f;
-    const int kv_head = a.kv_div > 1 ? kvh / a.kv_div : kvh;
-    const float *kb = a.k + (int64_t)kv_head * a.k_hs, *vb = a.v + (int64_t)kv_head * a.k_hs;
-    // K/V of a chunk pass through registers: the loads of chunk c0 + CH are
-    // issued before the MFMA work on chunk c0, so their latency overlaps it.
-    // Rows past the range repeat row blo (their scores are masked).
-    f32x4 kx[SV], vx[SV];
+    for (int c = wid; c < n_sub; c += NW) {
+        const bool more = c + NW < n_sub;
+        wait_vmcnt<L>();                        // the K tile has landed (V's loads are younger)
+        float4 kf[NST / 4];
 #pragma unroll
-    for (int u = 0; u < SV; u++) {
-        const int i = t + u * NTH, kk = i / (HD / 4), d4 = (i % (HD / 4)) * 4;
-        const int j = blo + kk < bhi ? blo + kk : blo;
-        kx[u] = *reinterpret_cast<const f32x4 *>(kb + (int64_t)j * a.k_rs + d4);
-        vx[u] = *reinterpret_cast<const f32x4 *>(vb + (int64_t)j * a.k_rs + d4);
-    }
-    for (int c0 = blo; c0 < bhi; c0 += CH) {
-        __syncthreads();
-        // stage keys [c0, c0 + CH)
-#pragma unroll
-        for (int u = 0; u < SV; u++) {
-            const int i = t + u * NTH, kk = i / (HD / 4), d4 = (i % (HD / 4)) * 4;
-            *reinterpret_cast<f32x4 *>(&Ks[kk][d4]) = kx[u];
-            *reinterpret_cast<f32x4 *>(&Vs[kk][d4]) = vx[u];
+        for (int s = 0; s < NST / 4; s++)
+            kf[s] = *reinterpret_cast<const float4 *>(Ks + lq * RB + (((lg * (NST / 4) + s) ^ (lq & 7)) * 16));
+        if (more) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            issue(kb, Ks, c + NW, true);
         }
-        __syncthreads();
-        // next chunk (past the last one: rows blo again, unused)
-#pragma unroll
-        for (int u = 0; u < SV; u++) {
-            const int i = t + u * NTH, kk = i / (HD / 4), d4 = (i % (HD / 4)) * 4;
-            const int j = c0 + CH + kk < bhi ? c0 + CH + kk : blo;
-            kx[u] = *reinterpret_cast<const f32x4 *>(kb + (int64_t)j * a.k_rs + d4);
-            vx[u] = *reinterpret_cast<const f32x4 *>(vb + (int64_t)j * a.k_rs + d4);
-        }
-        const int kt = 16 * ks;                 // this wave's sub-tile of the chunk
-        if (c0 + kt >= bhi) continue;
-        // S^T[key kt + 4 lg + i][query lq]
+        // S^T[key 4 lg + i][query lq]
         f32x4 st = {0.0f, 0.0f, 0.0f, 0.0f};
-        const float *kr = &Ks[kt + lq][lg * NST];
 #pragma unroll
         for (int s = 0; s < NST; s += 4) {
-            const float4 kx = *reinterpret_cast<const float4 *>(kr + s);
-            st = __builtin_amdgcn_mfma_f32_16x16x4f32(kx.x, qv[s], st, 0, 0, 0);
-            st = __builtin_amdgcn_mfma_f32_16x16x4f32(kx.y, qv[s + 1], st, 0, 0, 0);
-            st = __builtin_amdgcn_mfma_f32_16x16x4f32(kx.z, qv[s + 2], st, 0, 0, 0);
-            st = __builtin_amdgcn_mfma_f32_16x16x4f32(kx.w, qv[s + 3], st, 0, 0, 0);
+            st = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[s / 4].x, qv[s], st, 0, 0, 0);
+            st = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[s / 4].y, qv[s + 1], st, 0, 0, 0);
+            st = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[s / 4].z, qv[s + 2], st, 0, 0, 0);
+            st = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[s / 4].w, qv[s + 3], st, 0, 0, 0);
         }
         float sv[4], tm = -INFINITY;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int j = c0 + kt + 4 * lg + i;
+            const int j = blo + 16 * c + 4 * lg + i;
             sv[i] = (j >= lo && j < hi) ? __fmul_rn(st[i], a.scale) : -INFINITY;
             tm = fmaxf(tm, sv[i]);
         }
-        tm = fmaxf(tm, __shfl_xor(tm, 16, 64));
-        tm = fmaxf(tm, __shfl_xor(tm, 32, 64));
+        tm = xhalf_max(xrow16_max(tm));
         const float mn = fmaxf(m, tm);
         const float corr = (m == -INFINITY) ? 0.0f : expf(__fsub_rn(m, mn));
         float ps = 0.0f;
@@ -762,8 +765,7 @@ __device__ __forceinline__ void attn_mfma_block(const AttnRowsArgs &a, int q0) {
             sv[i] = sv[i] == -INFINITY ? 0.0f : expf(__fsub_rn(sv[i], mn));
         }
         ps = __fadd_rn(__fadd_rn(sv[0], sv[1]), __fadd_rn(sv[2], sv[3]));
-        ps = __fadd_rn(ps, __shfl_xor(ps, 16, 64));
-        ps = __fadd_rn(ps, __shfl_xor(ps, 32, 64));
+        ps = xhalf_sum(xrow16_sum(ps));
         l = fmaf(l, corr, ps);
         m = mn;
         // rescale the O rows this lane holds (queries 4 lg + j) by their owners' factors
@@ -774,47 +776,69 @@ __device__ __forceinline__ void attn_mfma_block(const AttnRowsArgs &a, int q0) {
         for (int n = 0; n < NT; n++)
 #pragma unroll
             for (int j = 0; j < 4; j++) o[n][j] = __fmul_rn(o[n][j], cj[j]);
-        // O += P V: step i pairs key kt + 4 lg + i of P (this lane's sv[i]) with V row kt + 4 lg + i
+        if (more) wait_vmcnt<L>();              // the V tile has landed (the next K's loads are younger)
+        else wait_vmcnt<0>();
+        float vf[4][NT];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float *vr = &Vs[kt + 4 * lg + i][lq];
+        for (int i = 0; i < 4; i++)
 #pragma unroll
-            for (int n = 0; n < NT; n++) o[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(sv[i], vr[16 * n], o[n], 0, 0, 0);
+            for (int n = 0; n < NT; n += 4) {
+                const float4 x = *reinterpret_cast<const float4 *>(Vs + (4 * lg + i) * RB + (lq * NT + n) * 4);
+                vf[i][n] = x.x; vf[i][n + 1] = x.y; vf[i][n + 2] = x.z; vf[i][n + 3] = x.w;
+            }
+        if (more) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            issue(vb, Vs, c + NW, false);
         }
+        // O += P V: step i pairs key 4 lg + i of P (this lane's sv[i]) with V row 4 lg + i
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int n = 0; n < NT; n++) o[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(sv[i], vf[i][n], o[n], 0, 0, 0);
     }
-    // merge the KS key splits of each head: (m, l) per query, O rows through LDS
-    __syncthreads();
-    float *Om = smem;                                   // [NW waves][16 rows][HD]
-    __shared__ float Mm[NW][16], Ll[NW][16];
+    // merge the NW key splits: (m, l) per query, O rows through LDS (every
+    // wave's loads have landed: its last wait was for all of them)
+    float *Om = reinterpret_cast<float *>(smem);           // [NW waves][16 rows][HD]
     if (lg == 0) { Mm[wid][lq] = m; Ll[wid][lq] = l; }
-#pragma unroll
-    for (int n = 0; n < NT; n++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) Om[(wid * 16 + 4 * lg + j) * HD + 16 * n + lq] = o[n][j];
     __syncthreads();
-    for (int i = t; i < G * 16 * HD; i += NTH) {
-        const int gg = i / (16 * HD), r = (i / HD) % 16, d = i % HD;
-        const int q = q0 + r;
-        if (q >= a.n_q) continue;
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int n = 0; n < NT; n += 4)
+            *reinterpret_cast<f32x4 *>(Om + (wid * 16 + 4 * lg + j) * HD + lq * NT + n) =
+                f32x4{o[n][j], o[n + 1][j], o[n + 2][j], o[n + 3][j]};
+    if (t < NW * 16) {
+        const int w = t >> 4, r = t & 15;
         float M = -INFINITY;
 #pragma unroll
-        for (int k2 = 0; k2 < KS; k2++) M = fmaxf(M, Mm[gg * KS + k2][r]);
-        float L = 0.0f, O = 0.0f;
+        for (int k2 = 0; k2 < NW; k2++) M = fmaxf(M, Mm[k2][r]);
+        Ff[w][r] = Mm[w][r] == -INFINITY ? 0.0f : expf(__fsub_rn(Mm[w][r], M));
+    }
+    __syncthreads();
+    for (int i = t; i < 16 * HD / 4; i += NW * 64) {
+        const int r = i / (HD / 4), d = (i % (HD / 4)) * 4;
+        const int q = q0 + r;
+        if (q >= a.n_q) continue;
+        float Ls = 0.0f;
+        f32x4 O = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int k2 = 0; k2 < KS; k2++) {
-            const int w = gg * KS + k2;
-            const float f = Mm[w][r] == -INFINITY ? 0.0f : expf(__fsub_rn(Mm[w][r], M));
-            L = fmaf(Ll[w][r], f, L);
-            O = fmaf(Om[(w * 16 + r) * HD + d], f, O);
+        for (int w = 0; w < NW; w++) {
+            const float f = Ff[w][r];
+            const f32x4 x = *reinterpret_cast<const f32x4 *>(Om + (w * 16 + r) * HD + d);
+            Ls = fmaf(Ll[w][r], f, Ls);
+#pragma unroll
+            for (int e = 0; e < 4; e++) O[e] = fmaf(x[e], f, O[e]);
         }
-        a.out[(int64_t)q * a.o_rs + (kvh * G + gg) * HD + d] = L > 0.0f ? __fdiv_rn(O, L) : 0.0f;
+        float *op = a.out + (int64_t)q * a.o_rs + h * HD + d;
+#pragma unroll
+        for (int e = 0; e < 4; e++) op[e] = Ls > 0.0f ? __fdiv_rn(O[e], Ls) : 0.0f;
     }
 }
 
-template <int HD, int G, int NW>
+template <int HD, int NW>
 __global__ __launch_bounds__(NW * 64) void k_attn_mfma(AttnRowsArgs a) {
     // causal: tiles in reverse, so that the blocks with the most keys start first
-    attn_mfma_block<HD, G, NW>(a, (a.window > 0 ? blockIdx.y : gridDim.y - 1 - blockIdx.y) * 16);
+    attn_mfma_block<HD, NW>(a, (a.window > 0 ? blockIdx.y : gridDim.y - 1 - blockIdx.y) * 16);
 }
 
 // Causal attention of several sequences in one launch (the multi-sequence
@@ -822,7 +846,7 @@ __global__ __launch_bounds__(NW * 64) void k_attn_mfma(AttnRowsArgs a) {
 // is that sequence's row block of a call of its own (the same q0, in the
 // same reverse order), with the sequence's query / output rows, KV cache,
 // key count and query offset.
-template <int HD, int G, int NW>
+template <int HD, int NW>
 __global__ __launch_bounds__(NW * 64) void k_attn_mfma_seqs(AttnSeqArgs s) {
     const int y = blockIdx.y;
     int b1 = s.blk[1];
@@ -848,7 +872,7 @@ __global__ __launch_bounds__(NW * 64) void k_attn_mfma_seqs(AttnSeqArgs s) {
     a.n_q = nq;
     a.n_k = nk;
     a.q_offset = qo;
-    attn_mfma_block<HD, G, NW>(a, (b1 - 1 - y) * 16);
+    attn_mfma_block<HD, NW>(a, (b1 - 1 - y) * 16);
 }
 
 hipError_t launch_attn_rows_seqs(const AttnSeqArgs &s0, int n_kv_heads, int head_dim, hipStream_t st) {
@@ -856,18 +880,16 @@ hipError_t launch_attn_rows_seqs(const AttnSeqArgs &s0, int n_kv_heads, int head
     if (s0.n < 1 || s0.n > QASR_ATTN_MAX_SEQ || a.window > 0 || head_dim != 128 || a.G != 2)
         return hipErrorInvalidValue;
     AttnSeqArgs s = s0;
-    s.base.kv_div = 1;
     s.blk[0] = 0;
     for (int j = 0; j < s.n; j++) {
         if (s.n_q[j] <= 0) return hipErrorInvalidValue;
         s.blk[j + 1] = s.blk[j] + (s.n_q[j] + 15) / 16;
     }
-    // both query heads of a KV head in one block of 16 waves, 8 key splits
-    // each: every head meets the key partition of launch_attn_rows' form for
-    // these heads (one head per 8-wave block, 8 splits; the same bits), and
-    // the block stages each K/V chunk once for the two heads
-    const dim3 grid(n_kv_heads, s.blk[s.n]);
-    hipLaunchKernelGGL((k_attn_mfma_seqs<128, 2, 16>), grid, dim3(1024), 0, st, s);
+    // launch_attn_rows' form for these heads (one query head per block, 8 key
+    // splits; the same bits)
+    s.base.kv_div = 2;
+    const dim3 grid(n_kv_heads * 2, s.blk[s.n]);
+    hipLaunchKernelGGL((k_attn_mfma_seqs<128, 8>), grid, dim3(512), 0, st, s);
     return hipGetLastError();
 }
 
@@ -875,22 +897,14 @@ hipError_t launch_attn_rows(const AttnRowsArgs &a, int n_kv_heads, int head_dim,
     if (a.G <= 0 || 32 % a.G != 0 || a.n_q <= 0) return hipErrorInvalidValue;
     const bool aligned = a.q_rs % 4 == 0 && a.k_rs % 4 == 0 && a.k_hs % 4 == 0 && (uintptr_t)a.q % 16 == 0 &&
                          (uintptr_t)a.k % 16 == 0 && (uintptr_t)a.v % 16 == 0;
-    if (aligned && (a.G == 1 || a.G == 2) && (head_dim == 128 || head_dim == 64)) {
-        const dim3 grid(n_kv_heads, (a.n_q + 15) / 16);
-        // 128-dim decoder heads (G = 2): one query head per block, its 8 waves
-        // 8 key splits (KV head x / 2); measured 30.0 us for the 404-row prefill
-        // against 32.5 with both heads of a KV head in one 8-wave block and 35.7
-        // with 4 waves.  64-dim encoder heads: 4 waves (12.4 us against 13.6 at 8).
-#define QAM(HDV, GV, NWV) hipLaunchKernelGGL((k_attn_mfma<HDV, GV, NWV>), grid, dim3(NWV * 64), 0, st, a);
-        if (head_dim == 128 && a.G == 2) {
-            AttnRowsArgs b = a;
-            b.kv_div = 2;
-            const dim3 grid1(n_kv_heads * 2, (a.n_q + 15) / 16);
-            hipLaunchKernelGGL((k_attn_mfma<128, 1, 8>), grid1, dim3(512), 0, st, b);
-        } else if (head_dim == 128) { QAM(128, 1, 8) }
-        else if (a.G == 2) { QAM(64, 2, 4) }
-        else { QAM(64, 1, 4) }
-#undef QAM
+    if (aligned && a.k_rs < 1 << 24 && (head_dim == 128 ? a.G <= 2 : head_dim == 64 && a.G == 1)) {
+        // one query head per block; the 128-dim heads' 8 waves are 8 key
+        // splits, the 64-dim encoder heads' 4
+        AttnRowsArgs b = a;
+        b.kv_div = a.G;
+        const dim3 grid(n_kv_heads * a.G, (a.n_q + 15) / 16);
+        if (head_dim == 128) hipLaunchKernelGGL((k_attn_mfma<128, 8>), grid, dim3(512), 0, st, b);
+        else hipLaunchKernelGGL((k_attn_mfma<64, 4>), grid, dim3(256), 0, st, b);
         return hipGetLastError();
     }
     const dim3 grid(n_kv_heads, (a.n_q + 32 / a.G - 1) / (32 / a.G));
