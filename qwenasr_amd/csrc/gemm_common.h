@@ -81,11 +81,20 @@ struct GeluRule {
     }
 };
 
-// the epilogue of 4 consecutive columns n .. n + 3 of row m (n % 4 == 0);
-// vec: C rows are 16-byte aligned
+// 4 consecutive floats p[n .. n + 3] of a row of N (n < N; repeats past the end)
+__device__ __forceinline__ f32x4 gemm_load4(const float *p, int n, int N, bool vec) {
+    if (vec && n + 3 < N) return *reinterpret_cast<const f32x4 *>(p + n);
+    f32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = p[min(n + e, N - 1)];
+    return v;
+}
+
+// the epilogue of 4 consecutive columns n .. n + 3 of row m (n % 4 == 0): b
+// holds their bias, c the old C (EPI_ACCUM); vec: C rows are 16-byte aligned
 template <int EPI>
-__device__ __forceinline__ void gemm_store4(const GemmArgs &g, const GeluRule &gr, int m, int n, f32x4 v, bool vec) {
-    const bool full = n + 3 < g.N;
+__device__ __forceinline__ void gemm_store4(const GemmArgs &g, const GeluRule &gr, int m, int n, f32x4 v, f32x4 b,
+                                            f32x4 c, bool vec) {
     if constexpr ((EPI & EPI_SWIGLU) != 0) {
         // columns (n, n + 1) are a (gate, up) pair: outputs n / 2, n / 2 + 1
         const int half = g.N >> 1, nv = half - half % 8;
@@ -101,18 +110,6 @@ __device__ __forceinline__ void gemm_store4(const GemmArgs &g, const GeluRule &g
         return;
     }
     float *cp = g.C + (int64_t)m * g.ldc + n;
-    f32x4 b = {0.0f, 0.0f, 0.0f, 0.0f}, c = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (full && vec) {
-        if (EPI & EPI_ACCUM) c = *reinterpret_cast<const f32x4 *>(cp);
-    } else {
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-            if ((EPI & EPI_ACCUM) && n + e < g.N) c[e] = cp[e];
-    }
-    if (g.bias) {
-#pragma unroll
-        for (int e = 0; e < 4; e++) b[e] = g.bias[min(n + e, g.N - 1)];
-    }
 #pragma unroll
     for (int e = 0; e < 4; e++) {
         if (EPI & EPI_ACCUM) {
@@ -127,7 +124,7 @@ __device__ __forceinline__ void gemm_store4(const GemmArgs &g, const GeluRule &g
             v[e] = gr(v[e], gidx);
         }
     }
-    if (full && vec) {
+    if (vec && n + 3 < g.N) {
         *reinterpret_cast<f32x4 *>(cp) = v;
     } else {
 #pragma unroll

@@ -156,6 +156,30 @@ __global__ __launch_bounds__(64 * S, 2) void k_gemm_ks(GemmArgs g) {
         for (int j = 0; j < WC; j++) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     const int fr = lane & 15, fg = lane >> 4;
     if (nst > 0) issue(0);
+    // The epilogue's operands (bias, the old C of +=) of this thread's runs of
+    // 4 columns are loaded ahead of the K loop: loaded behind it, every row
+    // group would wait for them and for the previous group's stores.
+    constexpr int Q = PR * (TN / 4), NQ = (Q + 64 * S - 1) / (64 * S);
+    const bool vec = (g.ldc & 3) == 0 && ((uintptr_t)g.C & 15) == 0;
+    constexpr bool HAS_B = (EPI & EPI_SWIGLU) == 0, HAS_C = (EPI & EPI_ACCUM) != 0;
+    // (run u of a thread keeps its column over the row groups; one column for all u when 64 S is a multiple of TN / 4)
+    constexpr int NB = 64 * S % (TN / 4) == 0 ? 1 : NQ;
+    f32x4 eb[NB], ec[HAS_C ? PH : 1][HAS_C ? NQ : 1];
+    auto ecol = [&](int u) { return min(n0 + ((t + u * 64 * S) % (TN / 4)) * 4, N - 1); };
+#pragma unroll
+    for (int u = 0; u < NB; u++) {
+        eb[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (HAS_B && g.bias) eb[u] = gemm_load4(g.bias, ecol(u), N, ((uintptr_t)g.bias & 15) == 0);
+    }
+    if constexpr (HAS_C) {
+#pragma unroll
+        for (int ph = 0; ph < PH; ph++)
+#pragma unroll
+            for (int u = 0; u < NQ; u++) {
+                const int m = min(m0 + ph * PR + (t + u * 64 * S) / (TN / 4), M - 1);
+                ec[ph][u] = gemm_load4(g.C + (int64_t)m * g.ldc, ecol(u), N, vec);
+            }
+    }
     __builtin_amdgcn_sched_barrier(0);
     for (int it = 0; it < nst; it += KU) {
         wait_vmcnt<0>();
@@ -207,8 +231,6 @@ __global__ __launch_bounds__(64 * S, 2) void k_gemm_ks(GemmArgs g) {
     // the S partial tiles meet in LDS, PR rows at a time; every thread then sums
     // the slices (in slice order) of its runs of 4 columns and finishes them
     float *P = reinterpret_cast<float *>(smem);
-    constexpr int Q = PR * (TN / 4), NQ = (Q + 64 * S - 1) / (64 * S);
-    const bool vec = (g.ldc & 3) == 0 && ((uintptr_t)g.C & 15) == 0;
     const GeluRule gr(g.gelu_n, (EPI & EPI_GELU) != 0);
 #pragma unroll
     for (int ph = 0; ph < PH; ph++) {
@@ -234,7 +256,8 @@ __global__ __launch_bounds__(64 * S, 2) void k_gemm_ks(GemmArgs g) {
                 for (int e = 0; e < 4; e++) v[e] = __fadd_rn(v[e], x[e]);
             }
             const int m = m0 + ph * PR + row, n = n0 + c4;
-            if (m < M && n < N) gemm_store4<EPI>(g, gr, m, n, v, vec);
+            if (m < M && n < N) gemm_store4<EPI>(g, gr, m, n, v, eb[NB > 1 ? u : 0],
+                                                ec[HAS_C ? ph : 0][HAS_C ? u : 0], vec);
         }
     }
 }
