@@ -629,6 +629,18 @@ __global__ __launch_bounds__(256) void k_attn_rows(AttnRowsArgs a) {
     }
 }
 
+// e^x for x <= 0 (the bf16-term softmax's x - max; -inf and NaN are the caller's): 2^(x
+// log2 e) with the product's rounding error and log2 e's second term carried to
+// first order, within 1.5 ulp, in half the operations of expf (whose range
+// checks have nothing to do here); results below 2^-126 become 0
+__device__ __forceinline__ float exp_neg(float x) {
+    constexpr float L = 0x1.715476p+0f, LL = 0x1.4ae0cp-26f;       // log2 e = L + LL
+    const float p = __fmul_rn(x, L);
+    const float r = fmaf(x, LL, fmaf(x, L, -p));
+    const float e = __builtin_amdgcn_exp2f(p);
+    return fmaf(e, __fmul_rn(r, 0x1.62e43p-1f), e);
+}
+
 // ---------------------------------------------------------------------------
 // The same multi-row attention on f32 MFMA (v_mfma_f32_16x16x4_f32, exact f32
 // products, f32 accumulation).  A block owns 16 query rows of one query head
@@ -841,13 +853,272 @@ __global__ __launch_bounds__(NW * 64) void k_attn_mfma(AttnRowsArgs a) {
     attn_mfma_block<HD, NW>(a, (a.window > 0 ? blockIdx.y : gridDim.y - 1 - blockIdx.y) * 16);
 }
 
+// ---------------------------------------------------------------------------
+// The decoder's prefill attention (128-dim heads, two query heads per KV head)
+// on bf16 MFMA: q, k, p and v are three bf16 terms each and a product is formed
+// from the six term pairs that matter (hi hi, hi mid, mid hi, mid mid, hi lo,
+// lo hi; the rest is below 2^-26 of it), accumulated in f32: f32-class like the
+// f32 MFMA form above, at 12 MFMAs of 16 clk for its 8 of 32.  The terms of a
+// K or V tile are formed once per wave, for the GH query heads (1 or 2) that
+// the block owns.
+//
+// Same streaming as above: 8 waves of their own 16-key sub-tiles, no barrier
+// before the merge.  Scores: S^T = K Q^T over 4 steps of 32 dims (lane l: key
+// or query l % 16, dims 32 s + 8 (l / 16) .. + 7).  O += P V contracts 16 keys
+// with 32-deep MFMAs, so each carries two term pairs: slots 0-3 of a lane are
+// its keys 4 (l / 16) + i with the first pair's terms, slots 4-7 the same keys
+// with the second's.
+//
+// What bounds it: per tile and two heads 96 MFMAs (1536 clk) and about 550
+// other vector operations (the term splits, the softmax).
+// ---------------------------------------------------------------------------
+// two pairs of f32 -> (hi, mid, lo), two packed dwords each
+__device__ __forceinline__ void split3_4(float x0, float x1, float x2, float x3, uint32_t (&hi)[2], uint32_t (&mi)[2],
+                                         uint32_t (&lo)[2], bf16x2 e0, bf16x2 e1) {
+    const float x[4] = {x0, x1, x2, x3};
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+        hi[e] = cvt_pk_bf16(x[2 * e], x[2 * e + 1]);
+        const bf16x2 h = __builtin_bit_cast(bf16x2, hi[e]);
+        const float r0 = __builtin_amdgcn_fdot2_f32_bf16(h, e0, x[2 * e], false);
+        const float r1 = __builtin_amdgcn_fdot2_f32_bf16(h, e1, x[2 * e + 1], false);
+        mi[e] = cvt_pk_bf16(r0, r1);
+        const bf16x2 m = __builtin_bit_cast(bf16x2, mi[e]);
+        lo[e] = cvt_pk_bf16(__builtin_amdgcn_fdot2_f32_bf16(m, e0, r0, false),
+                            __builtin_amdgcn_fdot2_f32_bf16(m, e1, r1, false));
+    }
+}
+
+template <int GH>
+__device__ __forceinline__ void attn_bf3_block(const AttnRowsArgs &a, int q0) {
+    constexpr int HD = 128, NW = 8, NT = HD / 16;
+    constexpr int RB = HD * 4, TB = 16 * RB, L = 8;
+    __shared__ __attribute__((aligned(16))) char smem[NW * 2 * TB];
+    __shared__ float Mm[NW][GH][16], Ll[NW][GH][16], Ff[NW][GH][16];
+    const int t = threadIdx.x, lane = t & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int h0 = blockIdx.x * GH;
+    const int lq = lane & 15, lg = lane >> 4;
+    const int qi = q0 + lq;
+    const int hi = qi < a.n_q ? min(a.q_offset + qi + 1, a.n_k) : 0;        // this lane's query sees keys [0, hi)
+    const int bhi = min(a.q_offset + min(q0 + 16, a.n_q), a.n_k);           // the block's keys
+    const int all = min(a.q_offset + q0 + 1, a.n_k);                        // keys that every query of the block sees
+    const bool full_rows = q0 + 16 <= a.n_q;
+    const int kv_head = h0 / 2;
+    const float *kb = a.k + (int64_t)kv_head * a.k_hs, *vb = a.v + (int64_t)kv_head * a.k_hs;
+    char *Ks = smem + wid * 2 * TB, *Vs = Ks + TB;
+    const int n_sub = (bhi + 15) / 16, lr = lane >> 5, ls = lane & 31;
+    auto issue = [&](const float *base, char *dst, int c, bool swz) {
+        const int j0 = 16 * c, last = bhi - 1 - j0;
+        const char *p = reinterpret_cast<const char *>(base + (int64_t)j0 * a.k_rs);
+#pragma unroll
+        for (int u = 0; u < L; u++) {
+            const int r = 2 * u + lr;
+            const uint32_t off = (uint32_t)min(r, last) * (uint32_t)a.k_rs * 4u + 16 * (swz ? ls ^ (r & 7) : ls);
+            lds_dma16_s(p, off, dst + 1024 * u);
+        }
+    };
+    if (wid < n_sub) {
+        issue(kb, Ks, wid, true);
+        issue(vb, Vs, wid, false);
+    }
+    uint32_t c0, c1;
+    asm("s_mov_b32 %0, 0xbf80" : "=s"(c0));
+    asm("s_mov_b32 %0, 0xbf800000" : "=s"(c1));
+    const bf16x2 e0 = __builtin_bit_cast(bf16x2, c0), e1 = __builtin_bit_cast(bf16x2, c1);
+    // the queries' terms: [head][step of 32 dims][term]
+    bf16x8 qf[GH][4][3];
+    {
+        float4 x[GH][4][2];
+#pragma unroll
+        for (int g = 0; g < GH; g++)
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const float *qp = a.q + (int64_t)min(qi, a.n_q - 1) * a.q_rs + (h0 + g) * HD + 32 * s + 8 * lg;
+                x[g][s][0] = *reinterpret_cast<const float4 *>(qp);
+                x[g][s][1] = *reinterpret_cast<const float4 *>(qp + 4);
+            }
+#pragma unroll
+        for (int g = 0; g < GH; g++)
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                split3(x[g][s][0], x[g][s][1], qf[g][s]);
+#pragma unroll
+                for (int e = 0; e < 3; e++) asm volatile("" : "+v"(qf[g][s][e]));   // formed here, not inside the loop
+            }
+    }
+    f32x4 o[GH][NT];
+    float m[GH], l[GH];
+#pragma unroll
+    for (int g = 0; g < GH; g++) {
+        m[g] = -INFINITY;
+        l[g] = 0.0f;
+#pragma unroll
+        for (int n = 0; n < NT; n++) o[g][n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    for (int c = wid; c < n_sub; c += NW) {
+        const bool more = c + NW < n_sub;
+        wait_vmcnt<L>();                        // the K tile has landed (V's loads are younger)
+        float4 kf[4][2];
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int e = 0; e < 2; e++)
+                kf[s][e] = *reinterpret_cast<const float4 *>(Ks + lq * RB + (((8 * s + 2 * lg + e) ^ (lq & 7)) * 16));
+        if (more) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            issue(kb, Ks, c + NW, true);
+        }
+        // S^T[key 4 lg + i][query lq] of each head, smallest terms first
+        f32x4 st[GH];
+#pragma unroll
+        for (int g = 0; g < GH; g++) st[g] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            bf16x8 kt[3];
+            split3(kf[s][0], kf[s][1], kt);
+#define QK(A, B) st[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[A], qf[g][s][B], st[g], 0, 0, 0);
+#pragma unroll
+            for (int g = 0; g < GH; g++) { QK(2, 0) }
+#pragma unroll
+            for (int g = 0; g < GH; g++) { QK(0, 2) }
+#pragma unroll
+            for (int g = 0; g < GH; g++) { QK(1, 1) }
+#pragma unroll
+            for (int g = 0; g < GH; g++) { QK(1, 0) }
+#pragma unroll
+            for (int g = 0; g < GH; g++) { QK(0, 1) }
+#pragma unroll
+            for (int g = 0; g < GH; g++) { QK(0, 0) }
+#undef QK
+        }
+        const bool masked = 16 * c + 16 > all || !full_rows;
+        bf16x8 pa[GH][3];                       // A operands of the three MFMAs per column tile
+#pragma unroll
+        for (int g = 0; g < GH; g++) {
+            float sv[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) sv[i] = __fmul_rn(st[g][i], a.scale);
+            if (masked) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) sv[i] = 16 * c + 4 * lg + i < hi ? sv[i] : -INFINITY;
+            }
+            const float tm = xhalf_max(xrow16_max(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]))));
+            const float mn = fmaxf(m[g], tm);
+            const float corr = (m[g] == -INFINITY) ? 0.0f : exp_neg(__fsub_rn(m[g], mn));
+#pragma unroll
+            for (int i = 0; i < 4; i++) sv[i] = sv[i] == -INFINITY ? 0.0f : exp_neg(__fsub_rn(sv[i], mn));
+            float ps = __fadd_rn(__fadd_rn(sv[0], sv[1]), __fadd_rn(sv[2], sv[3]));
+            ps = xhalf_sum(xrow16_sum(ps));
+            l[g] = fmaf(l[g], corr, ps);
+            m[g] = mn;
+            // rescale the O rows this lane holds (queries 4 lg + j) by their
+            // owners' factors, unless no query's maximum moved (factors 1)
+            if (__builtin_amdgcn_ballot_w64(corr != 1.0f) != 0) {
+                float cj[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) cj[j] = __shfl(corr, 4 * lg + j, 64);
+#pragma unroll
+                for (int n = 0; n < NT; n++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) o[g][n][j] = __fmul_rn(o[g][n][j], cj[j]);
+            }
+            uint32_t ph[2], pm[2], pl[2];
+            split3_4(sv[0], sv[1], sv[2], sv[3], ph, pm, pl, e0, e1);
+            pa[g][0] = __builtin_bit_cast(bf16x8, make_uint4(ph[0], ph[1], pl[0], pl[1]));   // with (lo, hi) of V
+            pa[g][1] = __builtin_bit_cast(bf16x8, make_uint4(pm[0], pm[1], pm[0], pm[1]));   // with (hi, mid)
+            pa[g][2] = __builtin_bit_cast(bf16x8, make_uint4(ph[0], ph[1], ph[0], ph[1]));   // with (hi, mid)
+        }
+        if (more) wait_vmcnt<L>();              // the V tile has landed (the next K's loads are younger)
+        else wait_vmcnt<0>();
+        // column lq of tile n is dim 8 lq + n: a lane's 8 dims of a V row are two slots
+        float4 vf[4][2];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int e = 0; e < 2; e++)
+                vf[i][e] = *reinterpret_cast<const float4 *>(Vs + (4 * lg + i) * RB + (2 * lq + e) * 16);
+        if (more) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            issue(vb, Vs, c + NW, false);
+        }
+#pragma unroll
+        for (int n = 0; n < NT; n++) {
+            uint32_t vh[2], vm[2], vl[2];
+            split3_4(vf[0][n >> 2][n & 3], vf[1][n >> 2][n & 3], vf[2][n >> 2][n & 3], vf[3][n >> 2][n & 3], vh, vm, vl,
+                     e0, e1);
+            const bf16x8 b0 = __builtin_bit_cast(bf16x8, make_uint4(vl[0], vl[1], vh[0], vh[1]));
+            const bf16x8 b1 = __builtin_bit_cast(bf16x8, make_uint4(vh[0], vh[1], vm[0], vm[1]));
+#pragma unroll
+            for (int g = 0; g < GH; g++) o[g][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa[g][0], b0, o[g][n], 0, 0, 0);
+#pragma unroll
+            for (int g = 0; g < GH; g++) o[g][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa[g][1], b1, o[g][n], 0, 0, 0);
+#pragma unroll
+            for (int g = 0; g < GH; g++) o[g][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa[g][2], b1, o[g][n], 0, 0, 0);
+        }
+    }
+    // merge the NW key splits: (m, l) per query, O rows through LDS (every
+    // wave's loads have landed: its last wait was for all of them)
+    float *Om = reinterpret_cast<float *>(smem);           // [NW waves][GH][16 rows][HD]
+#pragma unroll
+    for (int g = 0; g < GH; g++)
+        if (lg == 0) { Mm[wid][g][lq] = m[g]; Ll[wid][g][lq] = l[g]; }
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < GH; g++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int n = 0; n < NT; n += 4)
+                *reinterpret_cast<f32x4 *>(Om + ((wid * GH + g) * 16 + 4 * lg + j) * HD + lq * NT + n) =
+                    f32x4{o[g][n][j], o[g][n + 1][j], o[g][n + 2][j], o[g][n + 3][j]};
+    if (t < NW * GH * 16) {
+        const int w = t / (GH * 16), g = (t >> 4) % GH, r = t & 15;
+        float M = -INFINITY;
+#pragma unroll
+        for (int k2 = 0; k2 < NW; k2++) M = fmaxf(M, Mm[k2][g][r]);
+        Ff[w][g][r] = Mm[w][g][r] == -INFINITY ? 0.0f : exp_neg(__fsub_rn(Mm[w][g][r], M));
+    }
+    __syncthreads();
+    for (int i = t; i < GH * 16 * HD / 4; i += NW * 64) {
+        const int g = i / (16 * HD / 4), r = (i / (HD / 4)) % 16, d = (i % (HD / 4)) * 4;
+        const int q = q0 + r;
+        if (q >= a.n_q) continue;
+        float Ls = 0.0f;
+        f32x4 O = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            const float f = Ff[w][g][r];
+            const f32x4 x = *reinterpret_cast<const f32x4 *>(Om + ((w * GH + g) * 16 + r) * HD + d);
+            Ls = fmaf(Ll[w][g][r], f, Ls);
+#pragma unroll
+            for (int e = 0; e < 4; e++) O[e] = fmaf(x[e], f, O[e]);
+        }
+        float *op = a.out + (int64_t)q * a.o_rs + (h0 + g) * HD + d;
+#pragma unroll
+        for (int e = 0; e < 4; e++) op[e] = Ls > 0.0f ? __fdiv_rn(O[e], Ls) : 0.0f;
+    }
+}
+
+template <int GH>
+__global__ __launch_bounds__(512) void k_attn_bf3(AttnRowsArgs a) {
+    // tiles in reverse, so that the blocks with the most keys start first
+    attn_bf3_block<GH>(a, (gridDim.y - 1 - blockIdx.y) * 16);
+}
+
+// Both query heads of a KV head in one block (K and V terms formed once for the
+// two) where that leaves enough blocks: us with one / two heads per block, 672
+// blocks of two (1337 rows) 98.6 / 89.8, 208 (404 rows) 18.1 / 22.9, 40 (67
+// rows after 337) 13.6 / 21.8.
+static int attn_heads_per_block(int n_kv_heads, int64_t row_blocks) { return n_kv_heads * row_blocks >= 384 ? 2 : 1; }
+
 // Causal attention of several sequences in one launch (the multi-sequence
 // prefill): block row y belongs to sequence j (blk[j] <= y < blk[j + 1]) and
 // is that sequence's row block of a call of its own (the same q0, in the
 // same reverse order), with the sequence's query / output rows, KV cache,
 // key count and query offset.
-template <int HD, int NW>
-__global__ __launch_bounds__(NW * 64) void k_attn_mfma_seqs(AttnSeqArgs s) {
+template <int GH>
+__global__ __launch_bounds__(512) void k_attn_bf3_seqs(AttnSeqArgs s) {
     const int y = blockIdx.y;
     int b1 = s.blk[1];
     int64_t row = s.row[0];
@@ -872,7 +1143,7 @@ __global__ __launch_bounds__(NW * 64) void k_attn_mfma_seqs(AttnSeqArgs s) {
     a.n_q = nq;
     a.n_k = nk;
     a.q_offset = qo;
-    attn_mfma_block<HD, NW>(a, (b1 - 1 - y) * 16);
+    attn_bf3_block<GH>(a, (b1 - 1 - y) * 16);
 }
 
 hipError_t launch_attn_rows_seqs(const AttnSeqArgs &s0, int n_kv_heads, int head_dim, hipStream_t st) {
@@ -885,11 +1156,11 @@ hipError_t launch_attn_rows_seqs(const AttnSeqArgs &s0, int n_kv_heads, int head
         if (s.n_q[j] <= 0) return hipErrorInvalidValue;
         s.blk[j + 1] = s.blk[j] + (s.n_q[j] + 15) / 16;
     }
-    // launch_attn_rows' form for these heads (one query head per block, 8 key
-    // splits; the same bits)
-    s.base.kv_div = 2;
-    const dim3 grid(n_kv_heads * 2, s.blk[s.n]);
-    hipLaunchKernelGGL((k_attn_mfma_seqs<128, 8>), grid, dim3(512), 0, st, s);
+    // launch_attn_rows' form for these heads (the same bits for either number
+    // of heads per block)
+    if (attn_heads_per_block(n_kv_heads, s.blk[s.n]) == 2)
+        hipLaunchKernelGGL(k_attn_bf3_seqs<2>, dim3(n_kv_heads, s.blk[s.n]), dim3(512), 0, st, s);
+    else hipLaunchKernelGGL(k_attn_bf3_seqs<1>, dim3(n_kv_heads * 2, s.blk[s.n]), dim3(512), 0, st, s);
     return hipGetLastError();
 }
 
@@ -897,12 +1168,19 @@ hipError_t launch_attn_rows(const AttnRowsArgs &a, int n_kv_heads, int head_dim,
     if (a.G <= 0 || 32 % a.G != 0 || a.n_q <= 0) return hipErrorInvalidValue;
     const bool aligned = a.q_rs % 4 == 0 && a.k_rs % 4 == 0 && a.k_hs % 4 == 0 && (uintptr_t)a.q % 16 == 0 &&
                          (uintptr_t)a.k % 16 == 0 && (uintptr_t)a.v % 16 == 0;
+    const unsigned row_blocks = (unsigned)((a.n_q + 15) / 16);
+    if (aligned && a.k_rs < 1 << 24 && head_dim == 128 && a.G == 2 && a.window == 0) {
+        if (attn_heads_per_block(n_kv_heads, row_blocks) == 2)
+            hipLaunchKernelGGL(k_attn_bf3<2>, dim3(n_kv_heads, row_blocks), dim3(512), 0, st, a);
+        else hipLaunchKernelGGL(k_attn_bf3<1>, dim3(n_kv_heads * 2, row_blocks), dim3(512), 0, st, a);
+        return hipGetLastError();
+    }
     if (aligned && a.k_rs < 1 << 24 && (head_dim == 128 ? a.G <= 2 : head_dim == 64 && a.G == 1)) {
         // one query head per block; the 128-dim heads' 8 waves are 8 key
         // splits, the 64-dim encoder heads' 4
         AttnRowsArgs b = a;
         b.kv_div = a.G;
-        const dim3 grid(n_kv_heads * a.G, (a.n_q + 15) / 16);
+        const dim3 grid(n_kv_heads * a.G, row_blocks);
         if (head_dim == 128) hipLaunchKernelGGL((k_attn_mfma<128, 8>), grid, dim3(512), 0, st, b);
         else hipLaunchKernelGGL((k_attn_mfma<64, 4>), grid, dim3(256), 0, st, b);
         return hipGetLastError();
