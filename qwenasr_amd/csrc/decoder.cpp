@@ -274,6 +274,11 @@ int decoder_build(qasr_decoder *d, const qasr_dec_weights *w, const uint16_t *lm
     }
     TRY(dalloc(d, &d->token_log, d->max_seq));
     TRY(dalloc(d, &d->out_idx, 4));
+    if (hipHostMalloc((void **)&d->host_rep, 64, hipHostMallocDefault) != hipSuccess) {
+        d->host_rep = nullptr;
+        return qasr_fail(QASR_ERR_NOMEM, "decoder: pinned host allocation failed");
+    }
+    memset(d->host_rep, 0, 64);
     TRY(dalloc(d, &d->counters, QASR_COUNTERS));
     HIPCHK(hipMemsetAsync(d->counters, 0, QASR_COUNTERS * sizeof(unsigned), d->h->stream));
     TRY(dalloc(d, &d->am_val, QASR_ARGMAX_MAX_BLOCKS));
@@ -291,6 +296,7 @@ extern "C" void qasr_hip_decoder_free(qasr_decoder *d) {
     decoder_free_prefill(d);
     dbuf_release(d->head_out);
     if (d->lm_bf16) (void)hipFree(d->lm_bf16);
+    if (d->host_rep) (void)hipHostFree(d->host_rep);
     for (void *p : d->allocs) (void)hipFree(p);
     delete d;
 }
@@ -434,6 +440,7 @@ int decoder_enqueue_step(qasr_decoder *d, bool embed_mode, int only_kind) {
         am.state = d->state; am.token_log = d->token_log;
         am.rope_cos = d->rc; am.rope_sin = d->rs; am.rope_cur = d->rope_cur; am.max_pos = (int)d->max_seq;
         am.epoch = d->state + 4;
+        am.host_rep = d->step_report ? d->host_rep : nullptr;
         LAUNCHCHK(launch_argmax(am, true, argmax_blocks(d->lm_i8_rows), st, want(5), want(6)), "step argmax");
         if (want(6)) d->epochs += 1;
     }
@@ -441,7 +448,6 @@ int decoder_enqueue_step(qasr_decoder *d, bool embed_mode, int only_kind) {
 }
 
 int decoder_set_state(qasr_decoder *d, int32_t token) {
-    const int64_t hd = d->c.head_dim;
     // tags are epoch * 32 + layer in 32 bits: long before the epoch reaches
     // 2^27 (one call runs at most max_seq steps) the pairs are cleared and the
     // epoch restarts at 1
@@ -453,18 +459,10 @@ int decoder_set_state(qasr_decoder *d, int32_t token) {
         HIPCHK(hipStreamSynchronize(d->h->stream));
         d->epochs = 0;
     }
-    d->host_state[0] = token;
-    d->host_state[1] = (int32_t)d->len;
-    d->host_state[2] = 0;
-    d->host_state[3] = 0;
-    HIPCHK(hipMemcpyAsync(d->state, d->host_state, sizeof(d->host_state), hipMemcpyHostToDevice, d->h->stream));
     d->step_pos = d->len;
-    if (d->len < d->max_seq) {
-        HIPCHK(hipMemcpyAsync(d->rope_cur, d->rc + d->len * hd, sizeof(float) * hd, hipMemcpyDeviceToDevice,
-                              d->h->stream));
-        HIPCHK(hipMemcpyAsync(d->rope_cur + hd, d->rs + d->len * hd, sizeof(float) * hd, hipMemcpyDeviceToDevice,
-                              d->h->stream));
-    }
+    d->rep_valid = false;
+    LAUNCHCHK(launch_step_begin(d->state, token, (int)d->len, d->rc, d->rs, d->rope_cur, (int)d->max_seq, d->h->stream),
+              "step begin");
     return QASR_OK;
 }
 
@@ -485,11 +483,13 @@ static int run_step_graph(qasr_decoder *d, int64_t cap, int n) {
         const int64_t pos0 = d->step_pos;
         HIPCHK(hipStreamBeginCapture(d->h->stream, hipStreamCaptureModeThreadLocal));
         int rc = QASR_OK;
+        d->step_report = n == 1;
         for (int k = 0; k < n && rc == QASR_OK; k++) {
             rc = decoder_enqueue_step(d, true);
             d->step_pos += 1;
         }
         d->step_pos = pos0;
+        d->step_report = true;
         hipError_t e = hipStreamEndCapture(d->h->stream, &g);
         if (rc != QASR_OK) {
             if (g) (void)hipGraphDestroy(g);
@@ -552,10 +552,12 @@ extern "C" int qasr_hip_decoder_forward(qasr_decoder *d, const float *embed, int
     } else {
         TRY(decoder_run_embed_step(d));
     }
-    HIPCHK(hipMemcpyAsync(d->host_state, d->state, sizeof(d->host_state), hipMemcpyDeviceToHost, d->h->stream));
+    // the step reported its token, fault flag and logit to pinned host memory:
+    // one wait, no copies
     HIPCHK(hipStreamSynchronize(d->h->stream));
-    TRY(decoder_fault_check(d));
-    *token_out = d->host_state[0];
+    if (d->host_rep[2]) TRY(decoder_fault_check(d));
+    d->rep_valid = true;
+    *token_out = d->host_rep[0];
     d->len += 1;
     return QASR_OK;
 }
@@ -589,6 +591,10 @@ extern "C" int qasr_hip_decoder_generate(qasr_decoder *d, const float *first_emb
 extern "C" int qasr_hip_decoder_last_logit(qasr_decoder *d, float *best) {
     if (!d || !best) return qasr_fail(QASR_ERR_INVALID, "decoder_last_logit: null argument");
     CHECK_H(d->h);
+    if (d->rep_valid) {
+        memcpy(best, d->host_rep + 3, sizeof(float));
+        return QASR_OK;
+    }
     HIPCHK(hipMemcpyAsync(best, d->out_idx + 1, sizeof(float), hipMemcpyDeviceToHost, d->h->stream));
     HIPCHK(hipStreamSynchronize(d->h->stream));
     return QASR_OK;

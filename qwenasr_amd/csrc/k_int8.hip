@@ -375,7 +375,27 @@ __global__ __launch_bounds__(256) void k_argmax_finish(ArgmaxArgs a, int n_parts
             a.state[2] += 1;
         }
         if (a.epoch) a.epoch[0] += 1;
+        if (a.host_rep) {
+            a.host_rep[0] = tok;
+            a.host_rep[1] = next_pos;
+            a.host_rep[2] = a.state[5];
+            a.host_rep[3] = __float_as_int(bv);
+        }
     }
+}
+
+__global__ __launch_bounds__(256) void k_step_begin(int *state, int token, int pos, const float *__restrict__ rope_cos,
+                                                    const float *__restrict__ rope_sin, float *rope_cur, int max_pos) {
+    const int t = threadIdx.x;
+    if (pos < max_pos) rope_cur[t] = (t < 128 ? rope_cos : rope_sin)[(int64_t)pos * 128 + (t & 127)];
+    if (t < 4) state[t] = t == 0 ? token : t == 1 ? pos : 0;
+}
+
+hipError_t launch_step_begin(int *state, int token, int pos, const float *rope_cos, const float *rope_sin,
+                             float *rope_cur, int max_pos, hipStream_t st) {
+    hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(256), 0, st, state, token, pos, rope_cos, rope_sin, rope_cur,
+                       max_pos);
+    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------

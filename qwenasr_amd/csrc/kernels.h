@@ -54,8 +54,13 @@ struct ArgmaxArgs {
     float *rope_cur;          // nullable: receives the cos, sin rows of the next position
     int max_pos;
     int *epoch;               // nullable: advanced by one per decode step (the qkv + attention tags)
+    int *host_rep;            // nullable: pinned host memory that receives {token, position, fault, logit bits}
 };
 
+// starts a run of decode steps: state {token, pos, 0, 0} and, for pos < max_pos,
+// the RoPE rows (cos, sin) of pos
+hipError_t launch_step_begin(int *state, int token, int pos, const float *rope_cos, const float *rope_sin,
+                             float *rope_cur, int max_pos, hipStream_t st);
 hipError_t launch_pack_int8(const uint16_t *w, int64_t n, int K, int mode, int8_t *q, float *s,
                             hipStream_t st);
 hipError_t launch_quant_act(const float *x, int K, int8_t *q, float *xs, hipStream_t st);
