@@ -326,26 +326,36 @@ static void go_ks(GemmArgs g, hipStream_t st) {
 // costs from sweeps over M = 15 ... 1300 and the shapes of both models; e.g.
 // N = 1024, K = 2048: 16 x 32 tiles 4.9-5.0 us up to 256 of them (M = 67; 32 x
 // 64 7.9), 32 x 64 8.5 at M = 404 (32 x 32 11.0), 32 x 128 14.4 at M = 800
-// (32 x 64 17.3).  Plain rows prefer 64 x 64 tiles to 32 x 128: half the B
-// rows through LDS.
+// (32 x 64 17.3), 48 x 128 20.6 at M = 1300 (32 x 128 25.5); N = 6144, K = 1024
+// at M = 404 32 x 160 18.4 (32 x 64 20.8), N = 2688, K = 896 48 x 96 10.1 (10.9):
+// larger tiles move fewer bytes per product where they leave no last round
+// nearly empty.  Plain rows prefer 64 x 64 tiles to 32 x 128: half the B rows
+// through LDS.
 template <bool BP, int EPI>
 static void go_ks_rows(const GemmArgs &g, hipStream_t st) {
     if (g.N < 2048) {
-        static const KsForm f[] = {{16, 32, 30}, {32, 32, 45}, {32, 64, 65}, {32, 128, 105}};
+        static const KsForm f[] = {{16, 32, 30}, {32, 32, 45}, {32, 64, 65}, {48, 64, 85}, {32, 128, 105}, {48, 128, 165}};
         switch (ks_pick(f, g.M, g.N)) {
             case 0: go_ks<false, BP, EPI, 16, 32, 8, 2>(g, st); break;
             case 1: go_ks<false, BP, EPI, 32, 32, 8, 1>(g, st); break;
             case 2: go_ks<false, BP, EPI, 32, 64, 8, 1>(g, st); break;
-            default: go_ks<false, BP, EPI, 32, 128, 8, 1>(g, st); break;
+            case 3: go_ks<false, BP, EPI, 48, 64, 8, 1>(g, st); break;
+            case 4: go_ks<false, BP, EPI, 32, 128, 8, 1>(g, st); break;
+            default: go_ks<false, BP, EPI, 48, 128, 8, 1>(g, st); break;
         }
         return;
     }
     if constexpr (BP) {
-        static const KsForm f[] = {{16, 64, 26}, {32, 64, 40}, {32, 128, 70}};
+        static const KsForm f[] = {{16, 64, 26}, {32, 64, 40}, {48, 64, 54}, {32, 128, 70},
+                                   {48, 96, 78}, {32, 160, 85}, {48, 128, 95}};
         switch (ks_pick(f, g.M, g.N)) {
             case 0: go_ks<false, BP, EPI, 16, 64, 4, 2>(g, st); break;
             case 1: go_ks<false, BP, EPI, 32, 64, 4, 1>(g, st); break;
-            default: go_ks<false, BP, EPI, 32, 128, 4, 1>(g, st); break;
+            case 2: go_ks<false, BP, EPI, 48, 64, 4, 1>(g, st); break;
+            case 3: go_ks<false, BP, EPI, 32, 128, 4, 1>(g, st); break;
+            case 4: go_ks<false, BP, EPI, 48, 96, 4, 1>(g, st); break;
+            case 5: go_ks<false, BP, EPI, 32, 160, 4, 1>(g, st); break;
+            default: go_ks<false, BP, EPI, 48, 128, 4, 1>(g, st); break;
         }
     } else {
         static const KsForm f[] = {{16, 64, 28}, {32, 64, 43}, {64, 64, 70}};

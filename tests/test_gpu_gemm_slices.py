@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 # 8 K slices below 2048 columns, 4 from there on; fewer K-steps than slices;
 # partial row and column tiles of every form (16 x 32 ... 32 x 128, 64 x 64)
 SHAPES = [(1, 64, 32), (16, 1023, 512), (33, 2047, 96), (129, 1000, 2048), (600, 96, 1024), (2100, 1030, 64),
-          (15, 2048, 32), (40, 2050, 160), (300, 2303, 1024), (1500, 2049, 64), (700, 6150, 96)]
+          (15, 2048, 32), (40, 2050, 160), (300, 2303, 1024), (1500, 2049, 64), (700, 6150, 96), (404, 6144, 64), (390, 2690, 96),
+          (1300, 1030, 96), (790, 900, 160), (200, 2700, 64), (1300, 4100, 32)]
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
@@ -41,7 +42,8 @@ def test_linear_slices(dev, M, N, K):
 
 
 @pytest.mark.parametrize("hidden,inter,vocab,rows", [(64, 64, 33, 1), (192, 320, 1003, 17), (1024, 448, 2050, 70),
-                                                     (256, 192, 2047, 300)])
+                                                     (256, 192, 2047, 300), (64, 128, 6144, 404), (64, 64, 2690, 390),
+                                                     (64, 64, 2700, 200), (64, 64, 4100, 500)])
 def test_fragment_major_head(dev, hidden, inter, vocab, rows):
     """A separate head equal to the tied embedding (plain rows) gives its bits."""
     from qwenasr_amd.model import Decoder
