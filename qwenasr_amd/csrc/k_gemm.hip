@@ -206,6 +206,12 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(GemmArgs g) {
 // the wait count is the same in every iteration.  Requires K % 64 == 0 and
 // 16-byte aligned rows.
 //
+// VEC (N a multiple of 4, 16-byte aligned C rows): the columns are the MFMA's
+// rows, so a lane ends with 4 consecutive columns and stores 16 bytes (LM head at
+// M = 375 153 -> 143 us, the same bits).  Other N keep a column per lane: 16
+// consecutive floats per store, where 4 scalar stores of the other layout would
+// be 4 rows apart each (424 x 82070 x 1024 102 -> 144 us).
+//
 // KP > 1 splits the K loop inside the block: 4 KP waves in KP groups of 4,
 // group p taking the K-steps p, p + KP, ... through a ring of its own; at the
 // end groups 1 .. KP - 1 leave their partial tiles in LDS and group 0 adds
@@ -223,8 +229,8 @@ __device__ __attribute__((aligned(256))) int4 g_gemm_zero16[16];
 __device__ __forceinline__ int a_swz(int r) { return (r >> 1) & 7; }
 __device__ __forceinline__ int b_swz(int r) { return (r & 3) ^ ((r >> 2) & 3); }
 
-template <int NS, int BM, int BN, int KP>
-__global__ __launch_bounds__(256 * KP) void k_gemm_lds(GemmArgs g) {
+template <int NS, int BM, int BN, int KP, bool VEC>
+__global__ __launch_bounds__(256 * KP, BM * BN > 64 * 64 ? 2 : 1) void k_gemm_lds(GemmArgs g) {
     constexpr int BK = 64;
     constexpr int ASZ = BM * 128, BSZ = BN * 64, STG = ASZ + BSZ;
     constexpr int LA = BM / 32, LB = BN / 64;                        // one-KiB loads per wave per stage
@@ -232,8 +238,8 @@ __global__ __launch_bounds__(256 * KP) void k_gemm_lds(GemmArgs g) {
     // fragment (BN/4-column strips), so no fragment is converted twice.
     // (Measured and rejected for the LM head at M = 375: 2 x 2 waves of
     // (BM/2) x (BN/2), which halve the A reads from LDS but widen every B
-    // fragment in two waves: 189 -> 209 us with 128 x 128 tiles, 248 us with
-    // 128 x 256 tiles of one block per CU.)
+    // fragment in two waves: 143 -> 160 us with 128 x 128 tiles, 157-167 with
+    // 192 x 128 and 128 x 256; 8 waves on 128 x 256 tiles 156-162.)
     constexpr int WR = BM / 16, WC = BN / 4 / 16;
     static_assert(BM % 32 == 0 && BN % 64 == 0, "tile");
     static_assert((KP - 1) * 4 * WR * WC * 4 * 64 * 4 <= KP * NS * STG, "partials fit the rings");
@@ -283,20 +289,29 @@ __global__ __launch_bounds__(256 * KP) void k_gemm_lds(GemmArgs g) {
     // The column scales do not depend on the products: loaded before the
     // ring's first stage, so that no load is left after the K loop.  Being
     // older than every ring load, they are complete by the first wait.
-    float pre_s[WC];
+    const int fr = lane & 15, fg = lane >> 4;
+    f32x4 pre_s[WC];
     if (grp == 0) {
+        const bool sv = ((uintptr_t)g.scale & 15) == 0;
 #pragma unroll
-        for (int j = 0; j < WC; j++) pre_s[j] = g.scale[min(n0 + nw + j * 16 + (lane & 15), N - 1)];
+        for (int j = 0; j < WC; j++) {
+            if constexpr (VEC) {
+                pre_s[j] = gemm_load4(g.scale, min(n0 + nw + j * 16 + 4 * fg, N - 1), N, sv);
+            } else {
+                const float x = g.scale[min(n0 + nw + j * 16 + fr, N - 1)];
+                pre_s[j] = f32x4{x, x, x, x};
+            }
+        }
     }
 
 #pragma unroll
     for (int s = 0; s < NS - 1; s++) issue(s, s);
-    const int fr = lane & 15, fg = lane >> 4;
     for (int kt = 0; kt < nit; kt++) {
         wait_vmcnt<(LA + LB) * (NS - 2)>();   // this wave's loads of stage kt have landed
         __syncthreads();                      // ... and every wave's; stage kt - 1 is free
         issue((kt + NS - 1) % NS, kt + NS - 1);
         const char *st = smem[kt % NS];
+        if (BN == 128) __builtin_amdgcn_iglp_opt(1);   // LDS reads spread between the MFMAs (LM head 143 -> 141 us)
 #pragma unroll
         for (int s = 0; s < BK / 32; s++) {
             bf16x8 bfrag[WC];
@@ -321,7 +336,8 @@ __global__ __launch_bounds__(256 * KP) void k_gemm_lds(GemmArgs g) {
                 const bf16x8 af = *reinterpret_cast<const bf16x8 *>(st + r * 128 + ((4 * s + fg) ^ a_swz(r)) * 16);
 #pragma unroll
                 for (int j = 0; j < WC; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bfrag[j], acc[i][j], 0, 0, 0);
+                    acc[i][j] = VEC ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfrag[j], af, acc[i][j], 0, 0, 0)
+                                    : __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bfrag[j], acc[i][j], 0, 0, 0);
             }
         }
     }
@@ -356,31 +372,37 @@ __global__ __launch_bounds__(256 * KP) void k_gemm_lds(GemmArgs g) {
         }
     }
 
-    // epilogue: lane holds rows 4*(lane/16)+r, column lane%16 of each 16x16
-    // tile; every value first, then only stores under the bounds tests: an
-    // operand use inside a store's branch would make the compiler wait for
-    // all vector memory there, the previous stores included
-    float outv[WR][WC][4];
+    // epilogue: a lane holds 4 consecutive columns of one row of each 16 x 16
+    // tile (VEC), else 4 consecutive rows of one column; every value first,
+    // then only stores under the bounds tests: an operand use inside a store's
+    // branch would make the compiler wait for all vector memory there, the
+    // previous stores included
 #pragma unroll
     for (int i = 0; i < WR; i++)
 #pragma unroll
         for (int j = 0; j < WC; j++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                float v = __fmul_rn(acc[i][j][r], pre_s[j]);
+                float v = __fmul_rn(acc[i][j][r], pre_s[j][r]);
                 asm volatile("" : "+v"(v));
-                outv[i][j][r] = v;
+                acc[i][j][r] = v;
             }
 #pragma unroll
     for (int i = 0; i < WR; i++)
 #pragma unroll
-        for (int j = 0; j < WC; j++)
+        for (int j = 0; j < WC; j++) {
+            if constexpr (VEC) {                 // N % 4 == 0: whole runs
+                const int m = m0 + i * 16 + fr, n = n0 + nw + j * 16 + 4 * fg;
+                if (m < M && n < N) *reinterpret_cast<f32x4 *>(g.C + (int64_t)m * g.ldc + n) = acc[i][j];
+            } else {
+                const int n = n0 + nw + j * 16 + fr;
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int m = m0 + i * 16 + (lane >> 4) * 4 + r;
-                const int n = n0 + nw + j * 16 + (lane & 15);
-                if (m < M && n < N) g.C[(int64_t)m * g.ldc + n] = outv[i][j][r];
+                for (int r = 0; r < 4; r++) {
+                    const int m = m0 + i * 16 + fg * 4 + r;
+                    if (m < M && n < N) g.C[(int64_t)m * g.ldc + n] = acc[i][j][r];
+                }
             }
+        }
 }
 
 template <int ASRC, int BSRC>
@@ -396,30 +418,57 @@ static hipError_t go_gemm(const GemmArgs &g, int epi, hipStream_t st) {
     return hipGetLastError();
 }
 
-// bf16 A x int8 B.  64 x 64 tiles while they leave fewer than ~2 blocks per CU
-// (K-steps of 64: with at least 16 of them and at most 32 tile columns, 4 K
-// groups per block of 3 stages each; else one group of 4 stages).  Measured
-// at M = 375 (config 1, us per launch, KP 1 -> 4): k / v 7.7 -> 6.6, q 8.5 ->
-// 7.5, o 12.4 -> 9.2, down 17.1 -> 11.9; gate / up (48 tile columns, 288 blocks
-// of 16 waves for 256 CUs) 10.2 -> 12.2, so they keep one group.  Beyond, 128 x
-// 128 tiles: four times the MFMA work per K-step and barrier, with 2 stages of
-// 24 KiB, so that 3 blocks share a CU (LM head at M = 375, 3 stages -> 2: 174 ->
-// 155 us, the same bits).  Measured and rejected there: 128 x 256 tiles
-// (218-226 us); 2 waves of 64-column strips, which halve the A reads from LDS
-// but need 287 registers (206 us); the M tiles of one column strip grouped on
-// one XCD (162 us, against 155); each block walking every M tile of its strip
-// (205 us); and the activations split into three int8 planes on the int8 MFMA
-// (273-282 us: three bytes per activation through the ring and the LDS reads).
+// bf16 A x int8 B.  K groups: 64 x 64 tiles in at most 32 columns, with at
+// least 16 K-steps of 64, run 4 groups per block of 3 stages each (config 1 at M
+// = 375, us per launch, KP 1 -> 4: k / v 7.7 -> 6.6, q 8.5 -> 7.5, o 12.4 -> 9.2,
+// down 17.1 -> 11.9; gate / up, 48 tile columns: 10.2 -> 12.2).
+//
+// Otherwise the tile is free (an element's sum runs over the same K-steps in
+// the same order in every form) and the call takes the form with the least
+// estimated time: `one` for a CU's first tile, `more` for each further round
+// of tiles over the 256 CUs, halfway between the whole and the fractional
+// count of rounds (several blocks share a CU).  The figures are fits, in 0.1 us
+// at K = 1024, to a sweep over M = 16 ... 404 and N = 4096 ... 151936; one (64 x
+// 128) is raised for the longer K, where two 64 x 64 tiles are faster.  us per
+// launch with 64 x 64 tiles below 2048 of them and 128 x 128 beyond, then by
+// this rule: M = 16, N = 60001 17.2 -> 14.0, N = 151936 42.2 -> 27.0; M = 64, N
+// = 151936 46.6 -> 37.0; M = 90, N = 60001 36.6 -> 27.6; M = 140, N = 151936
+// 88.6 -> 65.4; M = 375, N = 20000 32.2 -> 24.0; M = 404, N = 151936 182 -> 170.
+// The 128-column forms keep a ring of 2 stages, so that more blocks share a CU
+// (LM head at M = 375, 128 x 128, 3 stages -> 2: 174 -> 155 us).  Measured and
+// rejected there: the M tiles of one column strip grouped on one XCD (162 us,
+// against 155); each block walking every M tile of its strip (205); non-temporal
+// stores of C (143 -> 147); the activations split into three int8 planes on the
+// int8 MFMA (273-282: three bytes per activation through the ring).
+struct W8Form { int bm, bn, one, more; };
+
+template <bool VEC>
 static hipError_t go_gemm_lds(const GemmArgs &g, hipStream_t st) {
     const int64_t small_blocks = (int64_t)((g.N + 63) / 64) * ((g.M + 63) / 64);
-    if (small_blocks >= 2048) {
-        const dim3 grid((g.N + 127) / 128, (g.M + 127) / 128);
-        hipLaunchKernelGGL((k_gemm_lds<2, 128, 128, 1>), grid, dim3(256), 0, st, g);
+    if (small_blocks < 2048 && g.K / 64 >= 16 && (g.N + 63) / 64 <= 32) {
+        hipLaunchKernelGGL((k_gemm_lds<3, 64, 64, 4, VEC>), dim3((g.N + 63) / 64, (g.M + 63) / 64), dim3(1024), 0, st, g);
         return hipGetLastError();
     }
-    const dim3 grid((g.N + 63) / 64, (g.M + 63) / 64);
-    if (g.K / 64 >= 16 && grid.x <= 32) hipLaunchKernelGGL((k_gemm_lds<3, 64, 64, 4>), grid, dim3(1024), 0, st, g);
-    else hipLaunchKernelGGL((k_gemm_lds<4, 64, 64, 1>), grid, dim3(256), 0, st, g);
+    static const W8Form f[] = {{32, 64, 64, 26}, {64, 64, 80, 37}, {64, 128, 125, 68},
+                               {96, 128, 118, 80}, {128, 128, 132, 96}, {160, 128, 147, 119}};
+    int best = 5;
+    int64_t best_cost = INT64_MAX;
+    for (int i = 0; i < 6; i++) {
+        const int64_t rows = (g.M + f[i].bm - 1) / f[i].bm, tiles = rows * ((g.N + f[i].bn - 1) / f[i].bn);
+        if (rows > 65535) continue;                  // the grid's y limit
+        const int64_t rounds = (tiles + 255) / 256;
+        const int64_t c = 512 * (int64_t)f[i].one + (rounds > 1 ? f[i].more * (tiles + 256 * rounds - 512) : 0);
+        if (c < best_cost) { best_cost = c; best = i; }
+    }
+    const dim3 grid((g.N + f[best].bn - 1) / f[best].bn, (g.M + f[best].bm - 1) / f[best].bm);
+    switch (best) {
+        case 0: hipLaunchKernelGGL((k_gemm_lds<4, 32, 64, 1, VEC>), grid, dim3(256), 0, st, g); break;
+        case 1: hipLaunchKernelGGL((k_gemm_lds<4, 64, 64, 1, VEC>), grid, dim3(256), 0, st, g); break;
+        case 2: hipLaunchKernelGGL((k_gemm_lds<2, 64, 128, 1, VEC>), grid, dim3(256), 0, st, g); break;
+        case 3: hipLaunchKernelGGL((k_gemm_lds<2, 96, 128, 1, VEC>), grid, dim3(256), 0, st, g); break;
+        case 4: hipLaunchKernelGGL((k_gemm_lds<2, 128, 128, 1, VEC>), grid, dim3(256), 0, st, g); break;
+        default: hipLaunchKernelGGL((k_gemm_lds<2, 160, 128, 1, VEC>), grid, dim3(256), 0, st, g); break;
+    }
     return hipGetLastError();
 }
 
@@ -447,7 +496,9 @@ hipError_t launch_gemm(const GemmArgs &g0, int asrc, int bsrc, int epi, hipStrea
         // the LDS ring takes whole stages and 16-byte aligned rows
         const bool ring = epi == EPI_SCALE && !g.bias && g.K % 64 == 0 && (g.lda * 2) % 16 == 0 && g.ldb % 16 == 0 &&
                           (uintptr_t)g.A % 16 == 0 && (uintptr_t)g.B % 16 == 0;
-        return ring ? go_gemm_lds(g, st) : go_gemm<A_BF16, B_I8>(g, epi, st);
+        if (!ring) return go_gemm<A_BF16, B_I8>(g, epi, st);
+        const bool vec = g.N % 4 == 0 && g.ldc % 4 == 0 && (uintptr_t)g.C % 16 == 0;
+        return vec ? go_gemm_lds<true>(g, st) : go_gemm_lds<false>(g, st);
     }
     if (asrc == A_BF16 && bsrc == B_BF16) return go_gemm<A_BF16, B_BF16>(g, epi, st);
     return hipErrorInvalidValue;
