@@ -89,8 +89,8 @@ struct MelTables {
     MelTables() : win(400), dft(13 * 25 * 2 * 256, 0.0f), filt(8 * 13 * 256, 0.0f) {
         const float PI = 3.14159265358979323846264338327950288f;
         for (int i = 0; i < 400; i++) win[i] = 0.5f * (1.0f - cosf(2.0f * PI * (float)i / 400.0f));
-        // slot (lane, j) of a step at 4 lane + j: column lane % 16, row 16 step + 4 j + lane / 16
-        auto slot = [](int col, int row) { return ((row & 3) * 16 + col) * 4 + (row >> 2 & 3); };
+        // slot (lane, j) of a step at 4 lane + j: column lane % 16, row 16 step + 4 (lane / 16) + j
+        auto slot = [](int col, int row) { return ((row >> 2 & 3) * 16 + col) * 4 + (row & 3); };
         for (int k = 0; k < 201; k++)
             for (int n = 0; n < 400; n++) {
                 const float a = 2.0f * PI * (float)k * (float)n / 400.0f;

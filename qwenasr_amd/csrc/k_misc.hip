@@ -1255,10 +1255,6 @@ hipError_t launch_attn_rows(const AttnRowsArgs &a, int n_kv_heads, int head_dim,
 // power spectrum in LDS.  Bound by the MFMAs: 26 x 100 of 32 clk per block, 8.7
 // us a block.  Before: five launches over frames, real and imaginary parts and
 // power in memory, the products as f32 FMA tiles: 109 us for 3000 frames.
-// MFMA j of a step contracts samples (then bins) 16 s + 4 j .. + 3, one per lane
-// group, in order: every sum is the chain over k from 0 that one thread would
-// form.  A row keeps sample n at mel_slot(n), so that a lane's four are 16 bytes.
-__device__ __forceinline__ int mel_slot(int n) { return (n & ~15) | (n & 3) * 4 | (n >> 2 & 3); }
 constexpr int MEL_FT = 16, MEL_FS = 404, MEL_PS = 212;     // frames per block, LDS row strides (conflict-free)
 __global__ __launch_bounds__(832) void k_mel(float *__restrict__ mel, const float *__restrict__ x, int64_t ns,
                                              const float *__restrict__ window, const float *__restrict__ dft,
@@ -1280,11 +1276,11 @@ __global__ __launch_bounds__(832) void k_mel(float *__restrict__ mel, const floa
     __syncthreads();
     for (int i = t; i < MEL_FT * 400; i += 832) {
         const int r = i / 400, n = i - 400 * r;
-        fr[r][mel_slot(n)] = __fmul_rn(xs[r * 160 + n], window[n]);
+        fr[r][n] = __fmul_rn(xs[r * 160 + n], window[n]);
     }
     __syncthreads();
     {
-        // step s, slot (lane, j): sample 16 s + 4 j + lane / 16
+        // step s, slot (lane, j): sample 16 s + 4 (lane / 16) + j
         const f32x4 *tab = reinterpret_cast<const f32x4 *>(dft) + (int64_t)wave * 25 * 128 + lane;
         f32x4 re = {0.0f, 0.0f, 0.0f, 0.0f}, im = re;
 #pragma unroll 5
@@ -1300,7 +1296,7 @@ __global__ __launch_bounds__(832) void k_mel(float *__restrict__ mel, const floa
         // frames 4 lg + j, bin 16 wave + lq (0 past bin 200)
 #pragma unroll
         for (int j = 0; j < 4; j++)
-            pw[4 * lg + j][mel_slot(16 * wave + lq)] = __fadd_rn(__fmul_rn(re[j], re[j]), __fmul_rn(im[j], im[j]));
+            pw[4 * lg + j][16 * wave + lq] = __fadd_rn(__fmul_rn(re[j], re[j]), __fmul_rn(im[j], im[j]));
     }
     __syncthreads();
     if (wave < 8) {

@@ -336,7 +336,7 @@ hipError_t launch_build_prompt(float *out, const uint16_t *embed, const int *tok
 // dft and filt are MFMA-ordered (mel_tables in encoder.cpp): dft [13 bin
 // groups][25 steps][cos, sin][64 lanes][4], filt [8 filter groups][13 steps][64
 // lanes][4], slot (lane, j) of step s holding column (bin or filter) lane % 16
-// of the group and sample or bin 16 s + 4 j + lane / 16
+// of the group and sample or bin 16 s + 4 (lane / 16) + j
 int64_t mel_blocks(int64_t nf);
 hipError_t launch_mel(float *mel, const float *x, int64_t ns, const float *window, const float *dft, const float *filt,
                       int nf, float *bmax, hipStream_t st);
