@@ -40,7 +40,7 @@ struct qasr_encoder {
     float *pe = nullptr;                        // sinusoidal PE [tokens_per_chunk][d_model]
     int tokens_per_chunk = 0;
     // mel tables
-    float *window = nullptr, *dft = nullptr, *filters = nullptr;   // dft and filters MFMA-ordered (launch_mel)
+    float *window = nullptr, *dft_cos = nullptr, *dft_sin = nullptr, *filters = nullptr;
     // scratch (grown on demand)
     size_t scratch_bytes = 0;
     char *scratch = nullptr;
@@ -81,45 +81,36 @@ static float mel_to_hz(float m) {                       // audio.rs:214-223
     return m >= 15.0f ? 1000.0f * expf(logstep * (m - 15.0f)) : 200.0f * m / 3.0f;
 }
 
-// The front end's tables: the window, and the DFT's cos / sin rows and the
-// filters in launch_mel's MFMA order.  They depend on nothing, so a process
-// forms them once (160,000 libm calls; an encoder's load 4 ms shorter).
-struct MelTables {
-    std::vector<float> win, dft, filt;
-    MelTables() : win(400), dft(13 * 25 * 2 * 256, 0.0f), filt(8 * 13 * 256, 0.0f) {
-        const float PI = 3.14159265358979323846264338327950288f;
-        for (int i = 0; i < 400; i++) win[i] = 0.5f * (1.0f - cosf(2.0f * PI * (float)i / 400.0f));
-        // slot (lane, j) of a step at 4 lane + j: column lane % 16, row 16 step + 4 (lane / 16) + j
-        auto slot = [](int col, int row) { return ((row >> 2 & 3) * 16 + col) * 4 + (row & 3); };
-        for (int k = 0; k < 201; k++)
-            for (int n = 0; n < 400; n++) {
-                const float a = 2.0f * PI * (float)k * (float)n / 400.0f;
-                float *step = &dft[(size_t)((k / 16) * 25 + n / 16) * 512 + slot(k % 16, n % 16)];
-                step[0] = cosf(a);
-                step[256] = sinf(a);
-            }
-        float fft[201], ff[130], fd[129];                    // audio.rs:225-262
-        for (int i = 0; i < 201; i++) fft[i] = (float)i * (16000.0f / 2.0f) / 200.0f;
-        const float mmin = hz_to_mel(0.0f), mmax = hz_to_mel(8000.0f);
-        for (int i = 0; i < 130; i++) ff[i] = mel_to_hz(mmin + (mmax - mmin) * (float)i / 129.0f);
-        for (int i = 0; i < 129; i++) {
-            fd[i] = ff[i + 1] - ff[i];
-            if (fd[i] == 0.0f) fd[i] = 1e-6f;
+static void mel_tables(std::vector<float> &win, std::vector<float> &ct, std::vector<float> &sn,
+                       std::vector<float> &filt) {
+    const float PI = 3.14159265358979323846264338327950288f;
+    win.resize(400);
+    for (int i = 0; i < 400; i++) win[i] = 0.5f * (1.0f - cosf(2.0f * PI * (float)i / 400.0f));
+    ct.resize(201 * 400);
+    sn.resize(201 * 400);
+    for (int k = 0; k < 201; k++)
+        for (int n = 0; n < 400; n++) {
+            const float a = 2.0f * PI * (float)k * (float)n / 400.0f;
+            ct[k * 400 + n] = cosf(a);
+            sn[k * 400 + n] = sinf(a);
         }
-        for (int m = 0; m < 128; m++) {
-            const float enorm = 2.0f / (ff[m + 2] - ff[m]);
-            for (int f = 0; f < 201; f++) {
-                const float down = (fft[f] - ff[m]) / fd[m];
-                const float up = (ff[m + 2] - fft[f]) / fd[m + 1];
-                filt[(size_t)((m / 16) * 13 + f / 16) * 256 + slot(m % 16, f % 16)] = fmaxf(fminf(down, up), 0.0f) * enorm;
-            }
+    float fft[201], ff[130], fd[129];                    // audio.rs:225-262
+    for (int i = 0; i < 201; i++) fft[i] = (float)i * (16000.0f / 2.0f) / 200.0f;
+    const float mmin = hz_to_mel(0.0f), mmax = hz_to_mel(8000.0f);
+    for (int i = 0; i < 130; i++) ff[i] = mel_to_hz(mmin + (mmax - mmin) * (float)i / 129.0f);
+    for (int i = 0; i < 129; i++) {
+        fd[i] = ff[i + 1] - ff[i];
+        if (fd[i] == 0.0f) fd[i] = 1e-6f;
+    }
+    filt.assign(128 * 201, 0.0f);
+    for (int m = 0; m < 128; m++) {
+        const float enorm = 2.0f / (ff[m + 2] - ff[m]);
+        for (int f = 0; f < 201; f++) {
+            const float down = (fft[f] - ff[m]) / fd[m];
+            const float up = (ff[m + 2] - fft[f]) / fd[m + 1];
+            filt[m * 201 + f] = fmaxf(fminf(down, up), 0.0f) * enorm;
         }
     }
-};
-
-static const MelTables &mel_tables() {
-    static const MelTables t;
-    return t;
 }
 
 // a weight matrix through the pinned staging ring
@@ -227,10 +218,12 @@ static int encoder_build(qasr_encoder *e, const qasr_enc_weights *w) {
                 pe[p * D + half + d] = cosf(a);
             }
         TRY(eupload(e, &e->pe, pe.data(), pe.size()));
-        const MelTables &mt = mel_tables();
-        TRY(eupload(e, &e->window, mt.win.data(), mt.win.size()));
-        TRY(eupload(e, &e->dft, mt.dft.data(), mt.dft.size()));
-        TRY(eupload(e, &e->filters, mt.filt.data(), mt.filt.size()));
+        std::vector<float> win, ct, sn, filt;
+        mel_tables(win, ct, sn, filt);
+        TRY(eupload(e, &e->window, win.data(), win.size()));
+        TRY(eupload(e, &e->dft_cos, ct.data(), ct.size()));
+        TRY(eupload(e, &e->dft_sin, sn.data(), sn.size()));
+        TRY(eupload(e, &e->filters, filt.data(), filt.size()));
         HIPCHK(hipStreamSynchronize(e->h->stream));
     }
     TRY(stg.finish());
@@ -521,11 +514,68 @@ int64_t mel_frames_for(int64_t n) {
 
 // mel_spectrogram on device samples; mel [128][frames]
 int mel_dev(qasr_encoder *e, const float *x, int64_t ns, float *mel, float *scratch) {
-    LAUNCHCHK(launch_mel(mel, x, ns, e->window, e->dft, e->filters, (int)mel_frames_for(ns), scratch, e->h->stream), "mel");
+    hipStream_t st = e->h->stream;
+    const int nf = (int)mel_frames_for(ns);
+    float *fr = scratch, *re = fr + (int64_t)nf * 400, *im = re + (int64_t)nf * 201;
+    float *pT = im + (int64_t)nf * 201, *bmax = pT + (int64_t)nf * 201;
+    LAUNCHCHK(launch_mel_frames(fr, x, ns, e->window, nf, st), "mel frames");
+    GemmArgs g{};
+    g.M = 201; g.N = nf; g.K = 400;
+    g.A = e->dft_cos; g.lda = 400; g.B = fr; g.ldb = 400; g.C = re; g.ldc = nf;
+    LAUNCHCHK(launch_gemm_f32(g, st), "mel dft");
+    g.A = e->dft_sin; g.C = im;
+    LAUNCHCHK(launch_gemm_f32(g, st), "mel dft");
+    LAUNCHCHK(launch_mel_power(pT, re, im, nf, st), "mel power");
+    g.M = 128; g.N = nf; g.K = 201;
+    g.A = e->filters; g.lda = 201; g.B = pT; g.ldb = 201; g.C = mel; g.ldc = nf;
+    LAUNCHCHK(launch_gemm_f32(g, st), "mel filterbank");
+    LAUNCHCHK(launch_mel_log_norm(mel, (int64_t)128 * nf, bmax, st), "mel log");
     return QASR_OK;
 }
 
-size_t mel_scratch_floats(int64_t nf) { return (size_t)mel_blocks(nf); }
+size_t mel_scratch_floats(int64_t nf) { return (size_t)nf * (400 + 3 * 201) + (size_t)(128 * nf / 256 + 2); }
+
+// mel_spectrogram of n device signals at once: the frames, the two DFT GEMMs,
+// the power and the filterbank GEMM over all their frames together (each f32
+// GEMM element is a sum over K in a fixed order, whatever the frame count),
+// then each mel copied out to mel[j] [128][frames_j] and log-normalised with
+// its own maximum.  scratch: mel_multi_scratch_floats(total frames, largest).
+int mel_dev_multi(qasr_encoder *e, int n, const float *const *x, const int64_t *ns, float *const *mel, float *scratch) {
+    hipStream_t st = e->h->stream;
+    int64_t tot = 0;
+    for (int j = 0; j < n; j++) tot += mel_frames_for(ns[j]);
+    float *fr = scratch, *re = fr + tot * 400, *im = re + tot * 201, *pT = im + tot * 201, *all = pT + tot * 201;
+    float *bmax = all + tot * 128;
+    int64_t off = 0;
+    for (int j = 0; j < n; j++) {
+        const int nf = (int)mel_frames_for(ns[j]);
+        LAUNCHCHK(launch_mel_frames(fr + off * 400, x[j], ns[j], e->window, nf, st), "mel frames");
+        off += nf;
+    }
+    GemmArgs g{};
+    g.M = 201; g.N = (int)tot; g.K = 400;
+    g.A = e->dft_cos; g.lda = 400; g.B = fr; g.ldb = 400; g.C = re; g.ldc = tot;
+    LAUNCHCHK(launch_gemm_f32(g, st), "mel dft");
+    g.A = e->dft_sin; g.C = im;
+    LAUNCHCHK(launch_gemm_f32(g, st), "mel dft");
+    LAUNCHCHK(launch_mel_power(pT, re, im, (int)tot, st), "mel power");
+    g.M = 128; g.N = (int)tot; g.K = 201;
+    g.A = e->filters; g.lda = 201; g.B = pT; g.ldb = 201; g.C = all; g.ldc = tot;
+    LAUNCHCHK(launch_gemm_f32(g, st), "mel filterbank");
+    off = 0;
+    for (int j = 0; j < n; j++) {
+        const int64_t nf = mel_frames_for(ns[j]);
+        HIPCHK(hipMemcpy2DAsync(mel[j], sizeof(float) * nf, all + off, sizeof(float) * tot, sizeof(float) * nf, 128,
+                                hipMemcpyDeviceToDevice, st));
+        LAUNCHCHK(launch_mel_log_norm(mel[j], 128 * nf, bmax, st), "mel log");
+        off += nf;
+    }
+    return QASR_OK;
+}
+
+size_t mel_multi_scratch_floats(int64_t total_frames, int64_t max_frames) {
+    return (size_t)total_frames * (400 + 3 * 201 + 128) + (size_t)(128 * max_frames / 256 + 2);
+}
 
 extern "C" int qasr_hip_mel(qasr_encoder *e, const float *samples, int64_t n, float *mel_out, int64_t *frames) {
     if (!e) return qasr_fail(QASR_ERR_INVALID, "encoder is null");

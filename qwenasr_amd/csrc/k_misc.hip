@@ -1245,88 +1245,51 @@ hipError_t launch_attn_rows(const AttnRowsArgs &a, int n_kv_heads, int head_dim,
 // ---------------------------------------------------------------------------
 // mel pieces (audio.rs:273-372)
 // ---------------------------------------------------------------------------
-// One launch from samples to log-mel (audio.rs:273-372): a block owns 16 frames,
-// cuts and windows them into LDS (reflect padding of 200), forms the 201-bin
-// DFT and then the 128 filters on f32 MFMA (v_mfma_f32_16x16x4_f32, exact f32
-// products, f32 sums) and takes log10(max(v, 1e-10)); the block's maximum goes
-// to bmax for k_mel_norm.  13 waves: wave p the cos and sin products of bins
-// 16 p .. + 15 (rows of frames from LDS, the tables MFMA-ordered in L2, 2 KiB
-// per step of 16 samples), then waves 0-7 the filters 16 w .. + 15 over the
-// power spectrum in LDS.  Bound by the MFMAs: 26 x 100 of 32 clk per block, 8.7
-// us a block.  Before: five launches over frames, real and imaginary parts and
-// power in memory, the products as f32 FMA tiles: 109 us for 3000 frames.
-constexpr int MEL_FT = 16, MEL_FS = 404, MEL_PS = 212;     // frames per block, LDS row strides (conflict-free)
-__global__ __launch_bounds__(832) void k_mel(float *__restrict__ mel, const float *__restrict__ x, int64_t ns,
-                                             const float *__restrict__ window, const float *__restrict__ dft,
-                                             const float *__restrict__ filt, int nf, float *__restrict__ bmax) {
-    constexpr int SPAN = (MEL_FT - 1) * 160 + 400;
-    __shared__ __attribute__((aligned(16))) float fr[MEL_FT][MEL_FS];
-    __shared__ __attribute__((aligned(16))) float xs[SPAN];
-    __shared__ __attribute__((aligned(16))) float pw[MEL_FT][MEL_PS];
-    __shared__ float red[8];
-    const int t = threadIdx.x, lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int64_t t0 = (int64_t)blockIdx.x * MEL_FT;
-    const int lq = lane & 15, lg = lane >> 4;
-    for (int i = t; i < SPAN; i += 832) {
-        const int64_t p = t0 * 160 + i;         // index into the padded signal
-        int64_t s = p < 200 ? 200 - p : p < 200 + ns ? p - 200 : ns - 2 - (p - 200 - ns);
-        xs[i] = s >= 0 && s < ns ? x[s] : 0.0f;
+// frames[t][n] = padded[t * 160 + n] * window[n], reflect padding of 200
+__global__ __launch_bounds__(256) void k_mel_frames(float *__restrict__ fr, const float *__restrict__ x, int64_t ns,
+                                                    const float *__restrict__ window, int nf) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (int64_t)nf * 400) return;
+    const int n = (int)(i % 400);
+    const int64_t t = i / 400;
+    const int64_t p = t * 160 + n;          // index into the padded signal
+    float v;
+    if (p < 200) {
+        const int64_t s = 200 - p;
+        v = s < ns ? x[s] : 0.0f;
+    } else if (p < 200 + ns) {
+        v = x[p - 200];
+    } else {
+        const int64_t s = ns - 2 - (p - 200 - ns);
+        v = s >= 0 ? x[s] : 0.0f;
     }
+    fr[i] = __fmul_rn(v, window[n]);
+}
+
+// powT[t][k] = re^2 + im^2 from re/im [k][t]
+__global__ __launch_bounds__(256) void k_mel_power(float *__restrict__ pT, const float *__restrict__ re,
+                                                   const float *__restrict__ im, int nf) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (int64_t)nf * 201) return;
+    const int k = (int)(i % 201);
+    const int64_t t = i / 201;
+    const float r = re[k * (int64_t)nf + t], m = im[k * (int64_t)nf + t];
+    pT[i] = __fadd_rn(__fmul_rn(r, r), __fmul_rn(m, m));
+}
+
+// log10(max(v, 1e-10)) in place and per-block maxima
+__global__ __launch_bounds__(256) void k_mel_log(float *__restrict__ mel, int64_t n, float *__restrict__ bmax) {
+    __shared__ float red[4];
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    float v = -1e30f;
+    if (i < n) {
+        v = log10f(fmaxf(mel[i], 1e-10f));
+        mel[i] = v;
+    }
+    v = wave_max_f32(v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    for (int i = t; i < MEL_FT * 400; i += 832) {
-        const int r = i / 400, n = i - 400 * r;
-        fr[r][n] = __fmul_rn(xs[r * 160 + n], window[n]);
-    }
-    __syncthreads();
-    {
-        // step s, slot (lane, j): sample 16 s + 4 (lane / 16) + j
-        const f32x4 *tab = reinterpret_cast<const f32x4 *>(dft) + (int64_t)wave * 25 * 128 + lane;
-        f32x4 re = {0.0f, 0.0f, 0.0f, 0.0f}, im = re;
-#pragma unroll 5
-        for (int s = 0; s < 25; s++) {
-            const f32x4 a = *reinterpret_cast<const f32x4 *>(&fr[lq][16 * s + 4 * lg]);
-            const f32x4 c = tab[s * 128], d = tab[s * 128 + 64];
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                re = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], c[j], re, 0, 0, 0);
-                im = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], d[j], im, 0, 0, 0);
-            }
-        }
-        // frames 4 lg + j, bin 16 wave + lq (0 past bin 200)
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            pw[4 * lg + j][16 * wave + lq] = __fadd_rn(__fmul_rn(re[j], re[j]), __fmul_rn(im[j], im[j]));
-    }
-    __syncthreads();
-    if (wave < 8) {
-        const f32x4 *tab = reinterpret_cast<const f32x4 *>(filt) + (int64_t)wave * 13 * 64 + lane;
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int s = 0; s < 13; s++) {
-            const f32x4 a = tab[s * 64], p = *reinterpret_cast<const f32x4 *>(&pw[lq][16 * s + 4 * lg]);
-#pragma unroll
-            for (int j = 0; j < 4; j++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], p[j], acc, 0, 0, 0);
-        }
-        // filters 16 wave + 4 lg + j, frame t0 + lq
-        float mx = -1e30f;
-        if (t0 + lq < nf) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const float v = log10f(fmaxf(acc[j], 1e-10f));
-                mel[(int64_t)(16 * wave + 4 * lg + j) * nf + t0 + lq] = v;
-                mx = fmaxf(mx, v);
-            }
-        }
-        mx = wave_max_f32(mx);
-        if (lane == 0) red[wave] = mx;
-    }
-    __syncthreads();
-    if (t == 0) {
-        float v = red[0];
-        for (int w = 1; w < 8; w++) v = fmaxf(v, red[w]);
-        bmax[blockIdx.x] = v;
-    }
+    if (threadIdx.x == 0) bmax[blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
 __global__ __launch_bounds__(256) void k_mel_norm(float *__restrict__ mel, int64_t n, const float *__restrict__ bmax,
@@ -1344,16 +1307,20 @@ __global__ __launch_bounds__(256) void k_mel_norm(float *__restrict__ mel, int64
         mel[i] = __fdiv_rn(__fadd_rn(fmaxf(mel[i], mn), 4.0f), 4.0f);
 }
 
-int64_t mel_blocks(int64_t nf) { return (nf + MEL_FT - 1) / MEL_FT; }
-
-hipError_t launch_mel(float *mel, const float *x, int64_t ns, const float *window, const float *dft, const float *filt,
-                      int nf, float *bmax, hipStream_t st) {
-    if (nf <= 0 || ns <= 0) return hipErrorInvalidValue;
-    const int nb = (int)mel_blocks(nf);
-    const int64_t n = (int64_t)128 * nf;
-    hipLaunchKernelGGL(k_mel, dim3(nb), dim3(832), 0, st, mel, x, ns, window, dft, filt, nf, bmax);
-    hipLaunchKernelGGL(k_mel_norm, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 1024)), dim3(256), 0, st, mel, n,
-                       bmax, nb);
+hipError_t launch_mel_frames(float *fr, const float *x, int64_t ns, const float *window, int nf, hipStream_t st) {
+    const int64_t n = (int64_t)nf * 400;
+    hipLaunchKernelGGL(k_mel_frames, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, fr, x, ns, window, nf);
+    return hipGetLastError();
+}
+hipError_t launch_mel_power(float *pT, const float *re, const float *im, int nf, hipStream_t st) {
+    const int64_t n = (int64_t)nf * 201;
+    hipLaunchKernelGGL(k_mel_power, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, pT, re, im, nf);
+    return hipGetLastError();
+}
+hipError_t launch_mel_log_norm(float *mel, int64_t n, float *bmax, hipStream_t st) {
+    const int nb = (int)((n + 255) / 256);
+    hipLaunchKernelGGL(k_mel_log, dim3(nb), dim3(256), 0, st, mel, n, bmax);
+    hipLaunchKernelGGL(k_mel_norm, dim3(std::min(nb, 1024)), dim3(256), 0, st, mel, n, bmax, nb);
     return hipGetLastError();
 }
 

@@ -241,6 +241,7 @@ hipError_t launch_gemm_ks(const GemmArgs &g, int asrc, int bsrc, int epi, hipStr
 inline bool gemm_frag_ok(int64_t K) { return K > 0 && K % 32 == 0 && K <= GEMM_FRAG_MAX_K; }
 inline int64_t gemm_frag_rows(int64_t N) { return (N + 15) / 16 * 16; }
 hipError_t launch_pack_frag(uint16_t *b, int64_t N, int64_t K, hipStream_t st);
+hipError_t launch_gemm_f32(const GemmArgs &g, hipStream_t st);
 }  // namespace qasr
 
 namespace qasr {
@@ -332,14 +333,9 @@ hipError_t launch_gather_rows(float *dst, const float *src, const int32_t *rows,
                               hipStream_t st);
 hipError_t launch_build_prompt(float *out, const uint16_t *embed, const int *toks, int n_head, const float *mid,
                                int n_mid, int n_tail, int H, hipStream_t st);
-// log-mel [128][nf] of one signal of ns samples; bmax: mel_blocks(nf) floats.
-// dft and filt are MFMA-ordered (mel_tables in encoder.cpp): dft [13 bin
-// groups][25 steps][cos, sin][64 lanes][4], filt [8 filter groups][13 steps][64
-// lanes][4], slot (lane, j) of step s holding column (bin or filter) lane % 16
-// of the group and sample or bin 16 s + 4 (lane / 16) + j
-int64_t mel_blocks(int64_t nf);
-hipError_t launch_mel(float *mel, const float *x, int64_t ns, const float *window, const float *dft, const float *filt,
-                      int nf, float *bmax, hipStream_t st);
+hipError_t launch_mel_frames(float *fr, const float *x, int64_t ns, const float *window, int nf, hipStream_t st);
+hipError_t launch_mel_power(float *pT, const float *re, const float *im, int nf, hipStream_t st);
+hipError_t launch_mel_log_norm(float *mel, int64_t n, float *bmax, hipStream_t st);
 hipError_t launch_head_norm_rope_strided(float *x, int64_t row_stride, const float *w, const float *cos_t,
                                          const float *sin_t, int64_t seq, int heads, float eps, int do_norm,
                                          int do_rope, hipStream_t st);

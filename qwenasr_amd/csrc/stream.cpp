@@ -221,7 +221,7 @@ static int encode_requests(qasr_decoder *d, qasr_encoder *e, std::vector<EncReq>
     if (live.empty()) return QASR_OK;
     TRY(dbuf_ensure(sc.audio, sizeof(float) * tot_s, enc_stream(d, e), d->h->stream));
     TRY(dbuf_ensure(sc.mel, sizeof(float) * 128 * tot_f, enc_stream(d, e), d->h->stream));
-    TRY(dbuf_ensure(sc.melsc, sizeof(float) * mel_scratch_floats(max_f), enc_stream(d, e), d->h->stream));
+    TRY(dbuf_ensure(sc.melsc, sizeof(float) * mel_multi_scratch_floats(tot_f, max_f), enc_stream(d, e), d->h->stream));
     std::vector<const float *> mels, xs;
     std::vector<float *> mels_w;
     std::vector<int64_t> frames, lens;
@@ -240,7 +240,7 @@ static int encode_requests(qasr_decoder *d, qasr_encoder *e, std::vector<EncReq>
         so += r.ns;
         fo += nf;
     }
-    for (size_t q = 0; q < live.size(); q++) TRY(mel_dev(e, xs[q], lens[q], mels_w[q], sc.melsc.as<float>()));
+    TRY(mel_dev_multi(e, (int)live.size(), xs.data(), lens.data(), mels_w.data(), sc.melsc.as<float>()));
     std::vector<int64_t> tok(live.size());
     if (live.size() == 1) {
         // one input: its rows straight into its destination
