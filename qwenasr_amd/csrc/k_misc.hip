@@ -1,6 +1,7 @@
 // Row-wise and element-wise kernels of the prefill, the audio encoder and the
 // mel front end, plus the multi-row (prefill / encoder-window) attention.
 #include <climits>
+#include <cfloat>
 #include <cstdlib>
 
 #include "kernels.h"
@@ -679,10 +680,12 @@ __global__ __launch_bounds__(256) void k_attn_rows(AttnRowsArgs a) {
     }
 }
 
-// e^x for x <= 0 (the bf16-term softmax's x - max; -inf and NaN are the caller's): 2^(x
-// log2 e) with the product's rounding error and log2 e's second term carried to
-// first order, within 1.5 ulp, in half the operations of expf (whose range
-// checks have nothing to do here); results below 2^-126 become 0
+// e^x for 0 >= x >= -2.36e38 (the bf16-term softmax's x - max): 2^(x log2 e) with
+// the product's rounding error and log2 e's second term carried to first order,
+// within 1.5 ulp, in half the operations of expf; results below 2^-126 become
+// 0.  Below that range (scores 2.36e38 or more apart) it is NaN, and the caller
+// forms the row again with expf; a cut-off here (fminf of the correction) cost
+// 2-5% of a short call's attention.
 __device__ __forceinline__ float exp_neg(float x) {
     constexpr float L = 0x1.715476p+0f, LL = 0x1.4ae0cp-26f;       // log2 e = L + LL
     const float p = __fmul_rn(x, L);
@@ -921,6 +924,16 @@ __global__ __launch_bounds__(NW * 64) void k_attn_mfma(AttnRowsArgs a) {
 //
 // What bounds it: per tile and two heads 96 MFMAs (1536 clk) and about 550
 // other vector operations (the term splits, the softmax).
+//
+// Its range is narrower than f32's: an infinite value, or one of 3.396e38 or
+// more (its bf16 rounding is infinite), has no three terms, and exp_neg has the
+// range above.  Each of these leaves NaN in what it meets.  And bf16's smallest
+// step is 2^-133: values of v below 2^-109 hold fewer than 24 bits.  So a row
+// whose merged sum or result is not finite, or below 2^-96 (but not 0), is formed
+// again in plain f32 by the wave that found it (only that row; the others keep
+// their bits).  What this does not see: a q or k value below 2^-109 against one
+// beyond 2^100, and weights below 2^-126 of the largest, which count as 0.
+// The check costs 0.2 us a call (16 rows 6.05 -> 6.25).
 // ---------------------------------------------------------------------------
 // two pairs of f32 -> (hi, mid, lo), two packed dwords each
 __device__ __forceinline__ void split3_4(float x0, float x1, float x2, float x3, uint32_t (&hi)[2], uint32_t (&mi)[2],
@@ -937,6 +950,38 @@ __device__ __forceinline__ void split3_4(float x0, float x1, float x2, float x3,
         lo[e] = cvt_pk_bf16(__builtin_amdgcn_fdot2_f32_bf16(m, e0, r0, false),
                             __builtin_amdgcn_fdot2_f32_bf16(m, e1, r1, false));
     }
+}
+
+// query q of head h (KV head kv_head, 128 dims) in f32 by one wave: a key per lane
+// for the scores, two dims per lane for the result
+__device__ __forceinline__ void attn_row_f32(const AttnRowsArgs &a, int q, int h, int kv_head, int lane) {
+    constexpr int HD = 128;
+    const float *qp = a.q + (int64_t)q * a.q_rs + h * HD;
+    const float *kb = a.k + (int64_t)kv_head * a.k_hs, *vb = a.v + (int64_t)kv_head * a.k_hs + 2 * lane;
+    const int hi = min(a.q_offset + q + 1, a.n_k);
+    float m = -INFINITY, l = 0.0f, o0 = 0.0f, o1 = 0.0f;
+    for (int j0 = 0; j0 < hi; j0 += 64) {
+        const int j = min(j0 + lane, hi - 1), n = min(64, hi - j0);
+        float s = 0.0f;
+        for (int d = 0; d < HD; d++) s = fmaf(qp[d], kb[(int64_t)j * a.k_rs + d], s);
+        s = lane < n ? __fmul_rn(s, a.scale) : -INFINITY;
+        const float mn = fmaxf(m, wave_max_f32(s));
+        const float corr = m == -INFINITY ? 0.0f : expf(__fsub_rn(m, mn));
+        const float p = s == -INFINITY ? 0.0f : expf(__fsub_rn(s, mn));
+        l = fmaf(l, corr, wave_sum_f32(p));
+        m = mn;
+        o0 = __fmul_rn(o0, corr);
+        o1 = __fmul_rn(o1, corr);
+        for (int k = 0; k < n; k++) {
+            const float pk = __shfl(p, k, 64);
+            const float *vp = vb + (int64_t)(j0 + k) * a.k_rs;
+            o0 = fmaf(pk, vp[0], o0);
+            o1 = fmaf(pk, vp[1], o1);
+        }
+    }
+    float *op = a.out + (int64_t)q * a.o_rs + h * HD + 2 * lane;
+    op[0] = l > 0.0f ? __fdiv_rn(o0, l) : 0.0f;
+    op[1] = l > 0.0f ? __fdiv_rn(o1, l) : 0.0f;
 }
 
 template <int GH>
@@ -1130,10 +1175,10 @@ __device__ __forceinline__ void attn_bf3_block(const AttnRowsArgs &a, int q0) {
         Ff[w][g][r] = Mm[w][g][r] == -INFINITY ? 0.0f : exp_neg(__fsub_rn(Mm[w][g][r], M));
     }
     __syncthreads();
+    // half a wave per row: each wave sees two whole rows a time
     for (int i = t; i < GH * 16 * HD / 4; i += NW * 64) {
         const int g = i / (16 * HD / 4), r = (i / (HD / 4)) % 16, d = (i % (HD / 4)) * 4;
         const int q = q0 + r;
-        if (q >= a.n_q) continue;
         float Ls = 0.0f;
         f32x4 O = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -1144,9 +1189,24 @@ __device__ __forceinline__ void attn_bf3_block(const AttnRowsArgs &a, int q0) {
 #pragma unroll
             for (int e = 0; e < 4; e++) O[e] = fmaf(x[e], f, O[e]);
         }
-        float *op = a.out + (int64_t)q * a.o_rs + (h0 + g) * HD + d;
+        bool ok = Ls > 0.0f;
 #pragma unroll
-        for (int e = 0; e < 4; e++) op[e] = Ls > 0.0f ? __fdiv_rn(O[e], Ls) : 0.0f;
+        for (int e = 0; e < 4; e++) {
+            O[e] = __fdiv_rn(O[e], Ls);
+            ok = ok && ((fabsf(O[e]) <= FLT_MAX && fabsf(O[e]) >= 0x1p-96f) || O[e] == 0.0f);
+        }
+        const uint64_t redo = __builtin_amdgcn_ballot_w64(!ok && q < a.n_q);
+        if ((lane < 32 ? (uint32_t)redo : (uint32_t)(redo >> 32)) == 0 && q < a.n_q) {
+            float *op = a.out + (int64_t)q * a.o_rs + (h0 + g) * HD + d;
+#pragma unroll
+            for (int e = 0; e < 4; e++) op[e] = O[e];
+        }
+        if (__builtin_expect(redo != 0, 0)) {
+            const int q2 = __builtin_amdgcn_readfirstlane(q);
+#pragma unroll 1
+            for (int u = 0; u < 2; u++)
+                if ((uint32_t)(redo >> (32 * u)) != 0) attn_row_f32(a, q2 + u, h0 + g, kv_head, lane);
+        }
     }
 }
 
