@@ -696,8 +696,8 @@ __device__ __forceinline__ float exp_neg(float x) {
 
 // ---------------------------------------------------------------------------
 // The same multi-row attention on f32 MFMA (v_mfma_f32_16x16x4_f32, exact f32
-// products, f32 accumulation).  A block owns 16 query rows of one query head
-// (KV head blockIdx.x / kv_div); its NW waves split the keys: wave w takes the
+// products, f32 accumulation): the encoder's windowed attention.  A block owns
+// 16 query rows of one head; its NW waves split the keys: wave w takes the
 // 16-key sub-tiles w, w + NW, ... with an online softmax of its own, and the NW
 // states are merged through LDS at the end.
 //
@@ -723,9 +723,8 @@ __device__ __forceinline__ float exp_neg(float x) {
 // LDS placement: slot q (16 bytes) of K row r sits at q ^ (r & 7): the 16 rows
 // of a fragment read fall in different banks; V rows are read along the row.
 // ---------------------------------------------------------------------------
-// One block's work: query rows [q0, q0 + 16) of query head blockIdx.x.
 template <int HD, int NW>
-__device__ __forceinline__ void attn_mfma_block(const AttnRowsArgs &a, int q0) {
+__global__ __launch_bounds__(NW * 64) void k_attn_mfma(AttnRowsArgs a) {
     constexpr int NST = HD / 4, NT = HD / 16;
     constexpr int RB = HD * 4, TB = 16 * RB;               // bytes of a K or V row, of a 16-key tile
     constexpr int LPR = RB / 16, RPL = 64 / LPR, L = 16 / RPL;   // lanes per row, rows per load, loads per tile
@@ -733,34 +732,23 @@ __device__ __forceinline__ void attn_mfma_block(const AttnRowsArgs &a, int q0) {
     __shared__ float Mm[NW][16], Ll[NW][16], Ff[NW][16];
     const int t = threadIdx.x, lane = t & 63;
     const int wid = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int h = blockIdx.x;
+    const int h = blockIdx.x, q0 = blockIdx.y * 16;
     const int lq = lane & 15, lg = lane >> 4;
     // key range of this lane's query (for the S^T masks) and of the block
     const int qi = q0 + lq;
-    // the block's sequence (windowed calls; blocks never straddle two)
+    // the block's sequence (blocks never straddle two)
     int s0 = 0, s1 = a.n_q;
-    if (a.window > 0) attn_sequence(a, q0, s0, s1);
+    attn_sequence(a, q0, s0, s1);
     int lo = 0, hi = 0;
     if (qi < a.n_q && qi < s1) {
-        if (a.window > 0) {
-            lo = s0 + ((qi - s0) / a.window) * a.window;
-            hi = min(lo + a.window, min(a.n_k, s1));
-        } else {
-            hi = min(a.q_offset + qi + 1, a.n_k);
-        }
+        lo = s0 + ((qi - s0) / a.window) * a.window;
+        hi = min(lo + a.window, min(a.n_k, s1));
     }
     const int qlast = min(q0 + 16, min(a.n_q, s1)) - 1;
     if (qlast < q0) return;                 // padding rows between two sequences
-    int blo, bhi;
-    if (a.window > 0) {
-        blo = s0 + ((q0 - s0) / a.window) * a.window;
-        bhi = min(s0 + ((qlast - s0) / a.window) * a.window + a.window, min(a.n_k, s1));
-    } else {
-        blo = 0;
-        bhi = min(a.q_offset + qlast + 1, a.n_k);
-    }
-    const int kv_head = a.kv_div > 1 ? h / a.kv_div : h;
-    const float *kb = a.k + (int64_t)kv_head * a.k_hs, *vb = a.v + (int64_t)kv_head * a.k_hs;
+    const int blo = s0 + ((q0 - s0) / a.window) * a.window;
+    const int bhi = min(s0 + ((qlast - s0) / a.window) * a.window + a.window, min(a.n_k, s1));
+    const float *kb = a.k + (int64_t)h * a.k_hs, *vb = a.v + (int64_t)h * a.k_hs;
     char *Ks = smem + wid * 2 * TB, *Vs = Ks + TB;
     // tile c (keys blo + 16 c ...): rows past the range repeat its last one (their scores are masked)
     const int n_sub = (bhi - blo + 15) / 16, lr = lane / LPR, ls = lane % LPR;
@@ -898,12 +886,6 @@ __device__ __forceinline__ void attn_mfma_block(const AttnRowsArgs &a, int q0) {
 #pragma unroll
         for (int e = 0; e < 4; e++) op[e] = Ls > 0.0f ? __fdiv_rn(O[e], Ls) : 0.0f;
     }
-}
-
-template <int HD, int NW>
-__global__ __launch_bounds__(NW * 64) void k_attn_mfma(AttnRowsArgs a) {
-    // causal: tiles in reverse, so that the blocks with the most keys start first
-    attn_mfma_block<HD, NW>(a, (a.window > 0 ? blockIdx.y : gridDim.y - 1 - blockIdx.y) * 16);
 }
 
 // ---------------------------------------------------------------------------
@@ -1285,14 +1267,12 @@ hipError_t launch_attn_rows(const AttnRowsArgs &a, int n_kv_heads, int head_dim,
         else hipLaunchKernelGGL(k_attn_bf3<1>, dim3(n_kv_heads * 2, row_blocks), dim3(512), 0, st, a);
         return hipGetLastError();
     }
-    if (aligned && a.k_rs < 1 << 24 && (head_dim == 128 ? a.G <= 2 : head_dim == 64 && a.G == 1)) {
-        // one query head per block; the 128-dim heads' 8 waves are 8 key
-        // splits, the 64-dim encoder heads' 4
-        AttnRowsArgs b = a;
-        b.kv_div = a.G;
-        const dim3 grid(n_kv_heads * a.G, row_blocks);
-        if (head_dim == 128) hipLaunchKernelGGL((k_attn_mfma<128, 8>), grid, dim3(512), 0, st, b);
-        else hipLaunchKernelGGL((k_attn_mfma<64, 4>), grid, dim3(256), 0, st, b);
+    if (aligned && a.k_rs < 1 << 24 && (head_dim == 128 || head_dim == 64) && a.G == 1 && a.window > 0) {
+        // one head per block; the 128-dim heads' 8 waves are 8 key splits, the
+        // 64-dim encoder heads' 4
+        const dim3 grid(n_kv_heads, row_blocks);
+        if (head_dim == 128) hipLaunchKernelGGL((k_attn_mfma<128, 8>), grid, dim3(512), 0, st, a);
+        else hipLaunchKernelGGL((k_attn_mfma<64, 4>), grid, dim3(256), 0, st, a);
         return hipGetLastError();
     }
     const dim3 grid(n_kv_heads, (a.n_q + 32 / a.G - 1) / (32 / a.G));

@@ -259,7 +259,6 @@ struct AttnRowsArgs {
     int q_offset;             // causal: query i sees keys [0, q_offset + i]
     int window;               // > 0: query i sees its window [w*window, min((w+1)*window, n_k))
     float scale;
-    int kv_div;               // set by the launchers: query head x reads KV head x / kv_div
     // windowed calls over several sequences (n_seg > 0): sequence j holds rows
     // [seg_lo[j], seg_hi[j]) and its windows start at seg_lo[j]; every seg_lo
     // is a multiple of 32, so no block of rows straddles two sequences and a
