@@ -292,8 +292,7 @@ static int egemm(qasr_encoder *e, const float *A, int64_t lda, const uint16_t *B
     g.M = M; g.N = N; g.K = K;
     g.A = A; g.lda = lda; g.B = B; g.ldb = ldb; g.C = C; g.ldc = ldc; g.bias = bias;
     g.gelu_n = gelu_n; g.gelu_rows = gelu_rows;
-    // (K slices go with the shape alone: a row's bits do not depend on how many
-    // rows, or sequences, share the call)
+    g.rows_alike = 1;                         // (a row's bits do not depend on how many sequences share the call)
     LAUNCHCHK(launch_gemm(g, A_F32_SPLIT, bsrc, epi, e->h->stream), "encoder gemm");
     return QASR_OK;
 }

@@ -263,6 +263,131 @@ __global__ __launch_bounds__(64 * S, 2) void k_gemm_ks(GemmArgs g) {
 }
 
 // ---------------------------------------------------------------------------
+// Plain rows of B with many tiles: a 128 x 128 tile per block whose four waves
+// share every K-step (32 rows of A each, all columns) through a ring of three
+// LDS stages, two in flight while one is computed, a block barrier per step.
+// Per product it moves half the bytes of the 64 x 64 tiles above, whose waves
+// each take whole K-steps; with few tiles those are faster, since they split
+// the K chain.  Past the last K-step the ring is filled with that step again,
+// so that the wait count is the same in every iteration.  VEC (16-byte aligned
+// C rows): the columns are the MFMA's rows, so a lane ends with 4 consecutive
+// columns; else a column per lane (16 consecutive floats per store).
+// ---------------------------------------------------------------------------
+template <int EPI, bool VEC>
+__global__ __launch_bounds__(256, 2) void k_gemm_ring(GemmArgs g) {
+    constexpr int T = 128, NS = 3, ASZ = T * 128, STG = ASZ + T * 64;
+    constexpr int LA = 4, LB = 2, WR = 2, WC = 8;                    // one-KiB loads per wave and stage; fragments
+    __shared__ __attribute__((aligned(16))) char smem[NS][STG];
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int M = g.M, N = g.N, m0 = blockIdx.y * T, n0 = blockIdx.x * T, nk = g.K / 32;
+    const char *A = reinterpret_cast<const char *>(g.A) + (int64_t)m0 * g.lda * 4;
+    const char *B = reinterpret_cast<const char *>(g.B) + (int64_t)n0 * g.ldb * 2;
+    uint32_t a_off[LA], b_off[LB];
+#pragma unroll
+    for (int u = 0; u < LA; u++) {
+        const int r = 8 * (wave * LA + u) + (lane >> 3), p = (lane & 7) ^ (r & 7);
+        a_off[u] = (uint32_t)min(r, M - 1 - m0) * (uint32_t)g.lda * 4u + 16 * p;
+    }
+#pragma unroll
+    for (int u = 0; u < LB; u++) {
+        const int r = 16 * (wave * LB + u) + (lane >> 2), p = (lane & 3) ^ ((r >> 1) & 3);
+        b_off[u] = (uint32_t)min(r, N - 1 - n0) * (uint32_t)g.ldb * 2u + 16 * p;
+    }
+    auto issue = [&](int buf, int kt) {
+        char *st = smem[buf];
+        const int kg = min(kt, nk - 1);
+        const char *ak = A + (int64_t)kg * 128, *bk = B + (int64_t)kg * 64;
+#pragma unroll
+        for (int u = 0; u < LA; u++) lds_dma16_s(ak, a_off[u], st + 1024 * (wave * LA + u));
+#pragma unroll
+        for (int u = 0; u < LB; u++) lds_dma16_s(bk, b_off[u], st + ASZ + 1024 * (wave * LB + u));
+    };
+    f32x4 acc[WR][WC];
+#pragma unroll
+    for (int i = 0; i < WR; i++)
+#pragma unroll
+        for (int j = 0; j < WC; j++) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const int fr = lane & 15, fg = lane >> 4, mw = m0 + 32 * wave;
+#pragma unroll
+    for (int s = 0; s < NS - 1; s++) issue(s, s);
+    for (int kt = 0; kt < nk; kt++) {
+        wait_vmcnt<(LA + LB) * (NS - 2)>();   // this wave's loads of stage kt have landed
+        __syncthreads();                      // ... and every wave's; stage kt - 1 is free
+        issue((kt + NS - 1) % NS, kt + NS - 1);
+        const char *st = smem[kt % NS];
+        bf16x8 xb[WC];
+#pragma unroll
+        for (int j = 0; j < WC; j++) {
+            const int n = j * 16 + fr;
+            xb[j] = *reinterpret_cast<const bf16x8 *>(st + ASZ + n * 64 + ((fg ^ ((n >> 1) & 3)) * 16));
+        }
+#pragma unroll
+        for (int i = 0; i < WR; i++) {
+            const int r = wave * 32 + i * 16 + fr;
+            bf16x8 af[3];
+            split3(*reinterpret_cast<const float4 *>(st + r * 128 + (((2 * fg) ^ (r & 7)) * 16)),
+                   *reinterpret_cast<const float4 *>(st + r * 128 + (((2 * fg + 1) ^ (r & 7)) * 16)), af);
+#pragma unroll
+            for (int a = 2; a >= 0; a--)
+#pragma unroll
+                for (int j = 0; j < WC; j++)
+                    acc[i][j] = VEC ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(xb[j], af[a], acc[i][j], 0, 0, 0)
+                                    : __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], xb[j], acc[i][j], 0, 0, 0);
+        }
+    }
+    wait_vmcnt<0>();                          // no load may land in LDS after the block ends
+    // the epilogue's operands (bias, the old C of +=), all of them ahead of the
+    // first store, behind which a load would wait for it
+    constexpr bool HAS_C = (EPI & EPI_ACCUM) != 0;
+    f32x4 eb[WC], ec[HAS_C ? WR : 1][HAS_C ? WC : 1];
+    const bool bv = ((uintptr_t)g.bias & 15) == 0;
+#pragma unroll
+    for (int j = 0; j < WC; j++) {
+        const int n = min(n0 + 16 * j + (VEC ? 4 * fg : fr), N - 1);
+        eb[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (g.bias) {
+            if (VEC) eb[j] = gemm_load4(g.bias, n, N, bv);
+            else eb[j][0] = g.bias[n];
+        }
+        if constexpr (HAS_C) {
+#pragma unroll
+            for (int i = 0; i < WR; i++) {
+                if (VEC) {
+                    ec[i][j] = gemm_load4(g.C + (int64_t)min(mw + 16 * i + fr, M - 1) * g.ldc, n, N, true);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        ec[i][j][r] = g.C[(int64_t)min(mw + 16 * i + 4 * fg + r, M - 1) * g.ldc + n];
+                }
+            }
+        }
+    }
+    const GeluRule gr(0, false);
+#pragma unroll
+    for (int i = 0; i < WR; i++)
+#pragma unroll
+        for (int j = 0; j < WC; j++) {
+            if constexpr (VEC) {
+                const int m = mw + 16 * i + fr, n = n0 + 16 * j + 4 * fg;
+                if (m < M && n < N)
+                    gemm_store4<EPI>(g, gr, m, n, acc[i][j], eb[j], ec[HAS_C ? i : 0][HAS_C ? j : 0], true);
+            } else {
+                const int n = n0 + 16 * j + fr;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int m = mw + 16 * i + 4 * fg + r;
+                    float v = acc[i][j][r], c = ec[HAS_C ? i : 0][HAS_C ? j : 0][r];
+                    if (HAS_C) v = __fadd_rn(g.bias ? __fadd_rn(c, eb[j][0]) : c, v);
+                    else if (g.bias) v = __fadd_rn(v, eb[j][0]);
+                    asm volatile("" : "+v"(v));              // formed here, not inside the store's branch
+                    if (m < M && n < N) g.C[(int64_t)m * g.ldc + n] = v;
+                }
+            }
+        }
+}
+
+// ---------------------------------------------------------------------------
 // B [N][K] bf16 rows -> fragment-major, in place: column group c (16 rows of
 // B) and K-step s (32 of K) are one KiB at (c K / 32 + s), in the order the
 // lanes of the MFMA's B operand hold it: lane l holds row l % 16, K 8 (l / 16)
@@ -301,9 +426,9 @@ hipError_t launch_pack_frag(uint16_t *b, int64_t N, int64_t K, hipStream_t st) {
 struct KsForm { int tm, tn, cost; };
 
 template <int NF>
-static int ks_pick(const KsForm (&f)[NF], int M, int N) {
+static int ks_pick(const KsForm (&f)[NF], int M, int N, int64_t &best_cost) {
     int best = 0;
-    int64_t best_cost = INT64_MAX;
+    best_cost = INT64_MAX;
     for (int i = 0; i < NF; i++) {
         const int64_t tiles = (int64_t)((M + f[i].tm - 1) / f[i].tm) * ((N + f[i].tn - 1) / f[i].tn);
         const int64_t c = (tiles + 255) / 256 * f[i].cost;
@@ -318,10 +443,26 @@ static void go_ks(GemmArgs g, hipStream_t st) {
     hipLaunchKernelGGL((k_gemm_ks<CONV, BP, EPI, TM, TN, S, KU>), dim3(tiles), dim3(64 * S), 0, st, g);
 }
 
-// Rows of f32.  The number of K slices depends on N alone, so that a row's
+// the ring's cost in ks_pick's units; a CU holds two of its tiles at a time
+static int64_t ring_cost(int M, int N) {
+    const int64_t rounds = ((int64_t)((M + 127) / 128) * ((N + 127) / 128) + 255) / 256;
+    return rounds / 2 * 380 + rounds % 2 * 320;
+}
+
+template <int EPI>
+static void go_ring(const GemmArgs &g, hipStream_t st) {
+    const dim3 grid((unsigned)((g.N + 127) / 128), (unsigned)((g.M + 127) / 128));
+    if (g.N % 4 == 0 && g.ldc % 4 == 0 && (uintptr_t)g.C % 16 == 0)
+        hipLaunchKernelGGL((k_gemm_ring<EPI, true>), grid, dim3(256), 0, st, g);
+    else hipLaunchKernelGGL((k_gemm_ring<EPI, false>), grid, dim3(256), 0, st, g);
+}
+
+// Rows of f32.  The number of K slices depends on N and K alone, so that a row's
 // result does not depend on how many rows share the call: 8 for N < 2048 (few
-// tiles: the K chain is what shortens), 4 above (8 partial tiles cost more
-// than they shorten: M = 404, N = 4096 15.5 against 12.8 us).  The tile is
+// tiles: the K chain is what shortens) from K = 512 on, else 4 (8 partial tiles
+// cost more than they shorten: M = 404, N = 4096 15.5 against 12.8 us; plain
+// rows, N = 1000, M = 1337, 8 -> 4 slices: K = 256 7.1 -> 6.1, K = 1024 13.3 ->
+// 13.5, and M = 16 there 3.6 -> 4.4).  The tile is
 // free (each element's sum runs over the same K-steps in the same order):
 // costs from sweeps over M = 15 ... 1300 and the shapes of both models; e.g.
 // N = 1024, K = 2048: 16 x 32 tiles 4.9-5.0 us up to 256 of them (M = 67; 32 x
@@ -331,11 +472,23 @@ static void go_ks(GemmArgs g, hipStream_t st) {
 // larger tiles move fewer bytes per product where they leave no last round
 // nearly empty.  Plain rows prefer 64 x 64 tiles to 32 x 128: half the B rows
 // through LDS.
+//
+// Plain rows take the ring where its estimate is less, unless the caller wants
+// rows alike (the ring adds the K-steps in one chain, so a row's bits would go
+// with the number of rows).  us, these forms / the ring: M = 2048, N = 12288,
+// K = 2048 432 / 243; M = 8192, N = 1024, K = 2048 131 / 88; M = 1600, N = 4096,
+// K = 1024 52 / 40; M = 1337, N = 4096 43 / 38 (taken from there on); M = 1337,
+// N = 6144 58 / 68; M = 404, N = 6144 22 / 29.
 template <bool BP, int EPI>
 static void go_ks_rows(const GemmArgs &g, hipStream_t st) {
-    if (g.N < 2048) {
+    int64_t cost;
+    const bool ring = !BP && !g.rows_alike && (g.M + 127) / 128 <= 65535;
+    if (g.N < 2048 && g.K >= 512) {
         static const KsForm f[] = {{16, 32, 30}, {32, 32, 45}, {32, 64, 65}, {48, 64, 85}, {32, 128, 105}, {48, 128, 165}};
-        switch (ks_pick(f, g.M, g.N)) {
+        const int best = ks_pick(f, g.M, g.N, cost);
+        if constexpr (!BP)
+            if (ring && ring_cost(g.M, g.N) <= cost) return go_ring<EPI>(g, st);
+        switch (best) {
             case 0: go_ks<false, BP, EPI, 16, 32, 8, 2>(g, st); break;
             case 1: go_ks<false, BP, EPI, 32, 32, 8, 1>(g, st); break;
             case 2: go_ks<false, BP, EPI, 32, 64, 8, 1>(g, st); break;
@@ -348,7 +501,7 @@ static void go_ks_rows(const GemmArgs &g, hipStream_t st) {
     if constexpr (BP) {
         static const KsForm f[] = {{16, 64, 26}, {32, 64, 40}, {48, 64, 54}, {32, 128, 70},
                                    {48, 96, 78}, {32, 160, 85}, {48, 128, 95}};
-        switch (ks_pick(f, g.M, g.N)) {
+        switch (ks_pick(f, g.M, g.N, cost)) {
             case 0: go_ks<false, BP, EPI, 16, 64, 4, 2>(g, st); break;
             case 1: go_ks<false, BP, EPI, 32, 64, 4, 1>(g, st); break;
             case 2: go_ks<false, BP, EPI, 48, 64, 4, 1>(g, st); break;
@@ -359,7 +512,9 @@ static void go_ks_rows(const GemmArgs &g, hipStream_t st) {
         }
     } else {
         static const KsForm f[] = {{16, 64, 28}, {32, 64, 43}, {64, 64, 70}};
-        switch (ks_pick(f, g.M, g.N)) {
+        const int best = ks_pick(f, g.M, g.N, cost);
+        if (ring && ring_cost(g.M, g.N) <= cost) return go_ring<EPI>(g, st);
+        switch (best) {
             case 0: go_ks<false, BP, EPI, 16, 64, 4, 2>(g, st); break;
             case 1: go_ks<false, BP, EPI, 32, 64, 4, 1>(g, st); break;
             default: go_ks<false, BP, EPI, 64, 64, 4, 1>(g, st); break;
@@ -374,7 +529,8 @@ static void go_ks_rows(const GemmArgs &g, hipStream_t st) {
 template <int EPI>
 static void go_ks_conv(const GemmArgs &g, hipStream_t st) {
     static const KsForm f[] = {{16, 32, 80}, {32, 32, 138}, {32, 64, 175}, {32, 96, 255}, {64, 96, 440}, {32, 160, 330}};
-    switch (ks_pick(f, g.M, g.N)) {
+    int64_t cost;
+    switch (ks_pick(f, g.M, g.N, cost)) {
         case 0: go_ks<true, true, EPI, 16, 32, 8, 2>(g, st); break;
         case 1: go_ks<true, true, EPI, 32, 32, 8, 1>(g, st); break;
         case 2: go_ks<true, true, EPI, 32, 64, 8, 1>(g, st); break;
@@ -385,7 +541,7 @@ static void go_ks_conv(const GemmArgs &g, hipStream_t st) {
 }
 
 // whole K-steps, 16-byte aligned rows, 32-bit offsets inside a tile (at most
-// 64 rows of A, 160 of B), a tile count that fits the grid
+// 128 rows of A, 160 of B), a tile count that fits the grid
 bool gemm_ks_ok(const GemmArgs &g, int asrc, int bsrc, int epi) {
     const int64_t tiles = (int64_t)((g.M + 15) / 16) * ((g.N + 31) / 32);
     if (g.K % 32 != 0 || (uintptr_t)g.A % 16 != 0 || (uintptr_t)g.B % 16 != 0 || tiles >= 1ll << 31) return false;

@@ -229,6 +229,7 @@ struct GemmArgs {
     int conv_hin, conv_win, conv_c, conv_hout, conv_wout, conv_kh, conv_kw, conv_sy, conv_sx, conv_py, conv_px;
     float conv_rc, conv_rkw;  // 1 / conv_c, 1 / conv_kw (set by the launcher)
     int m_major;              // tile order of k_gemm_ks (set by the launcher)
+    int rows_alike;           // f32 A: a row's bits must not depend on how many rows share the call
 };
 
 hipError_t launch_gemm(const GemmArgs &g, int asrc, int bsrc, int epi, hipStream_t st);

@@ -38,14 +38,14 @@ static int ensure_prefill(qasr_decoder *d, int64_t S) {
     return QASR_OK;
 }
 
-// The f32-class GEMMs slice K by the shape alone, so that a row's result is the
+// K is sliced by the shape alone (rows_alike), so that a row's result is the
 // same whether its sequence is prefilled alone or with others.  The layers'
 // weights and a separate head are fragment-major, the tied embedding is rows.
 static int gemm(qasr_decoder *d, const float *A, int64_t lda, const uint16_t *B, int64_t ldb, float *C,
                 int64_t ldc, int M, int N, int K, int epi, int bsrc = B_BF16_FRAG) {
     GemmArgs g{};
     g.M = M; g.N = N; g.K = K;
-    g.A = A; g.lda = lda; g.B = B; g.ldb = ldb; g.C = C; g.ldc = ldc;
+    g.A = A; g.lda = lda; g.B = B; g.ldb = ldb; g.C = C; g.ldc = ldc; g.rows_alike = 1;
     LAUNCHCHK(launch_gemm(g, A_F32_SPLIT, bsrc, epi, d->h->stream), "prefill gemm");
     return QASR_OK;
 }

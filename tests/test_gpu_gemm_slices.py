@@ -60,3 +60,31 @@ def test_fragment_major_head(dev, hidden, inter, vocab, rows):
     own = d.prefill_logits(emb)
     d.close()
     assert np.isfinite(tied).all() and (tied == own).all()
+
+
+# the ring of 128 x 128 tiles that plain rows take with many tiles: partial row and
+# column tiles, vector (N % 4 == 0) and scalar stores, one to 32 K-steps
+RING = [(4000, 2003, 32), (4000, 2004, 96), (1600, 4100, 1024), (8190, 1022, 512)]
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("M,N,K", RING)
+def test_linear_ring(dev, M, N, K, accumulate):
+    from qwenasr_amd import kernels as Kr
+    print(f"linear ring M={M} N={N} K={K} accumulate={accumulate}", flush=True)
+    r = rng(M * 7 + N * 3 + K)
+    x = r.normal(0, 1, (M, K)).astype(np.float32)
+    w = bf16(r.normal(0, 0.02, (N, K)))
+    b = r.normal(0, 1, N).astype(np.float32)
+    y0 = np.zeros((M + 1, N), np.float32)
+    if accumulate:
+        y0[:M] = r.normal(0, 1, (M, N))
+    y = dev.upload(y0)
+    Kr.linear(y, dev.upload(x), dev.upload(w), dev.upload(b), M, K, N, accumulate=accumulate)
+    got = y.numpy()
+    xd, wd = x.astype(np.float64), bf16f(w).astype(np.float64)
+    exact = xd @ wd.T + b + y0[:M]
+    # K + 2 roundings of partial sums no larger than sum |x w| + |b| + |y0|, each at most 2^-24
+    bound = (K + 2) * 2.0 ** -24 * (np.abs(xd) @ np.abs(wd).T + np.abs(b) + np.abs(y0[:M]))
+    assert (np.abs(got[:M] - exact) <= bound).all()
+    assert (got[M] == 0).all()                       # nothing past the last row
