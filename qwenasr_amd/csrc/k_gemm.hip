@@ -208,9 +208,9 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(GemmArgs g) {
 // the wait count is the same in every iteration.  Requires K % 64 == 0 and
 // 16-byte aligned rows.
 //
-// VEC (N a multiple of 4, 16-byte aligned C rows): the columns are the MFMA's
-// rows, so a lane ends with 4 consecutive columns and stores 16 bytes (LM head at
-// M = 375 153 -> 143 us, the same bits).  Other N keep a column per lane: 16
+// VEC (N a multiple of 4, 16-byte aligned C rows, K >= 512): the columns are the
+// MFMA's rows, so a lane ends with 4 consecutive columns and stores 16 bytes (the
+// same bits).  Other N keep a column per lane: 16
 // consecutive floats per store, where 4 scalar stores of the other layout would
 // be 4 rows apart each (424 x 82070 x 1024 102 -> 144 us).
 //
@@ -476,7 +476,11 @@ static hipError_t go_gemm(const GemmArgs &g, int epi, hipStream_t st) {
 // of tiles over the 256 CUs, halfway between the whole and the fractional
 // count of rounds (several blocks share a CU).  The figures are fits, in 0.1 us
 // at K = 1024, to a sweep over M = 16 ... 404 and N = 4096 ... 151936; one (64 x
-// 128) is raised for the longer K, where two 64 x 64 tiles are faster.  us per
+// 128) is raised for K = 2048 and 3072, where two 64 x 64 tiles are faster.  K <
+// 512, where a tile's fixed part weighs more, has figures of its own and stores a
+// column per lane (256 x 20000 x 192 11.3 -> 9.1 us, 375 x 60000 x 256 32.2 ->
+// 28.3 by both).  A third row for K from 1536 on was fitted too: 0.5%
+// faster on average over 262 shapes, the LM head at M = 375 3% slower.  us per
 // launch with 64 x 64 tiles below 2048 of them and 128 x 128 beyond, then by
 // this rule: M = 16, N = 60001 17.2 -> 14.0, N = 151936 42.2 -> 27.0; M = 64, N
 // = 151936 46.6 -> 37.0; M = 90, N = 60001 36.6 -> 27.6; M = 140, N = 151936
@@ -496,8 +500,11 @@ static hipError_t go_gemm_lds(const GemmArgs &g, hipStream_t st) {
         hipLaunchKernelGGL((k_gemm_lds<3, 64, 64, 4, VEC>), dim3((g.N + 63) / 64, (g.M + 63) / 64), dim3(1024), 0, st, g);
         return hipGetLastError();
     }
-    static const W8Form f[] = {{32, 64, 64, 26}, {64, 64, 80, 37}, {64, 128, 125, 68},
-                               {96, 128, 118, 80}, {128, 128, 132, 96}, {160, 128, 147, 119}};
+    static const W8Form longk[] = {{32, 64, 64, 26}, {64, 64, 80, 37}, {64, 128, 125, 68},
+                                   {96, 128, 118, 80}, {128, 128, 132, 96}, {160, 128, 147, 119}};
+    static const W8Form shortk[] = {{32, 64, 66, 27}, {64, 64, 94, 30}, {64, 128, 123, 59},
+                                    {96, 128, 143, 71}, {128, 128, 169, 88}, {160, 128, 176, 172}};
+    const W8Form *f = g.K < 512 ? shortk : longk;
     int best = 5;
     int64_t best_cost = INT64_MAX;
     for (int i = 0; i < 6; i++) {
@@ -544,7 +551,7 @@ hipError_t launch_gemm(const GemmArgs &g0, int asrc, int bsrc, int epi, hipStrea
         const bool ring = epi == EPI_SCALE && !g.bias && g.K % 64 == 0 && (g.lda * 2) % 16 == 0 && g.ldb % 16 == 0 &&
                           (uintptr_t)g.A % 16 == 0 && (uintptr_t)g.B % 16 == 0;
         if (!ring) return go_gemm<A_BF16, B_I8>(g, epi, st);
-        const bool vec = g.N % 4 == 0 && g.ldc % 4 == 0 && (uintptr_t)g.C % 16 == 0;
+        const bool vec = g.K >= 512 && g.N % 4 == 0 && g.ldc % 4 == 0 && (uintptr_t)g.C % 16 == 0;
         return vec ? go_gemm_lds<true>(g, st) : go_gemm_lds<false>(g, st);
     }
     if (asrc == A_BF16 && bsrc == B_BF16) return go_gemm<A_BF16, B_BF16>(g, epi, st);
