@@ -52,3 +52,56 @@ def test_w8_shapes_reach_every_form():
         seen.setdefault((f, K < 512), set()).add(vec)
     tiles = [(32, 64), (64, 64), (64, 128), (96, 128), (128, 128), (160, 128)]
     assert seen == {**{(t, False): {False, True} for t in tiles + ["K groups"]}, **{(t, True): {False} for t in tiles}}
+
+
+def ks_tables():
+    src = source("k_gemm_ks.hip")
+    t = [rows_of(x, 3) for x in re.findall(r"static const KsForm f\[\] = \{(.*?)\};", src, re.S)]
+    assert [len(x) for x in t] == [6, 7, 3, 6]       # rows: 8 slices; 4 slices fragment-major, plain; convolutions
+    two, one = (int(v) for v in re.search(r"return rounds / 2 \* (\d+) \+ rounds % 2 \* (\d+);", src).groups())
+    return t, two, one
+
+
+def ks_form(M, N, K, frag, alike):
+    """go_ks_rows' choice: (slices, rows, columns) or "ring"."""
+    t, two, one = ks_tables()
+    eight = N < 2048 and K >= 512
+    forms = t[0] if eight else t[1] if frag else t[2]
+
+    def cost(f):
+        return up(up(M, f[0]) * up(N, f[1]), 256) * f[2]
+    best = min(forms, key=cost)
+    rounds = up(up(M, 128) * up(N, 128), 256)
+    if not frag and not alike and rounds // 2 * two + rounds % 2 * one <= cost(best):
+        return "ring"
+    return (8 if eight else 4,) + best[:2]
+
+
+def test_linear_shapes_reach_every_plain_form():
+    from test_gpu_gemm_slices import EPILOGUE, RING
+    t, _, _ = ks_tables()
+    seen = set()
+    for M, N, K in EPILOGUE:
+        f = ks_form(M, N, K, False, False)
+        assert M % f[1] and N % f[2], (M, N, K, f)   # partial rows and columns
+        seen.add(f)
+    assert seen == {(8,) + f[:2] for f in t[0]} | {(4,) + f[:2] for f in t[2]}
+    assert all(ks_form(M, N, K, False, False) == "ring" and M % 128 and N % 128 for M, N, K in RING)
+
+
+def test_prefill_shapes_reach_every_fragment_major_form():
+    from test_gpu_gemm_slices import ALIKE
+    t, _, _ = ks_tables()
+    want = {1024: {(8,) + f[:2] for f in t[0]}, 2048: {(4,) + f[:2] for f in t[1]}}
+    for hidden, inter, rows in ALIKE:
+        # o_proj and down (+=) each reach every form of their width
+        for K in (2048, inter):
+            assert {ks_form(M, hidden, K, True, True) for M in rows} == want[hidden], (hidden, K)
+
+
+def test_encoder_shapes_reach_every_convolution_form():
+    from test_gpu_gemm_slices import CONV
+    t, _, _ = ks_tables()
+    forms = t[3]
+    seen = {min(forms, key=lambda f: up(up(800 * k, f[0]) * up(C, f[1]), 256) * f[2]) for C, k in CONV}
+    assert seen == set(forms)

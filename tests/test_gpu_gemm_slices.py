@@ -11,8 +11,8 @@ from conftest import bf16, bf16f, rng
 
 pytestmark = pytest.mark.gpu
 
-# 8 K slices below 2048 columns, 4 from there on; fewer K-steps than slices;
-# partial row and column tiles of every form (16 x 32 ... 32 x 128, 64 x 64)
+# 8 K slices below 2048 columns from K = 512 on, else 4; fewer K-steps than slices;
+# partial row and column tiles (every form: EPILOGUE and ALIKE below)
 SHAPES = [(1, 64, 32), (16, 1023, 512), (33, 2047, 96), (129, 1000, 2048), (600, 96, 1024), (2100, 1030, 64),
           (15, 2048, 32), (40, 2050, 160), (300, 2303, 1024), (1500, 2049, 64), (700, 6150, 96), (404, 6144, 64), (390, 2690, 96),
           (1300, 1030, 96), (790, 900, 160), (200, 2700, 64), (1300, 4100, 32)]
@@ -88,3 +88,75 @@ def test_linear_ring(dev, M, N, K, accumulate):
     bound = (K + 2) * 2.0 ** -24 * (np.abs(xd) @ np.abs(wd).T + np.abs(b) + np.abs(y0[:M]))
     assert (np.abs(got[:M] - exact) <= bound).all()
     assert (got[M] == 0).all()                       # nothing past the last row
+
+
+# bias and += in every plain-row form with partial rows and columns: 8 slices (K >=
+# 512) in 16 x 32 ... 48 x 128 tiles, 4 slices in 16 x 64, 32 x 64, 64 x 64
+# (test_gemm_forms.py holds the list to the dispatch's rule)
+EPILOGUE = [(45, 1003, 544), (135, 1010, 512), (404, 1000, 544), (600, 1000, 512), (900, 900, 544), (1300, 1030, 512),
+            (45, 2050, 544), (200, 2303, 96), (700, 2310, 160), (300, 1990, 96)]
+
+
+@pytest.mark.parametrize("M,N,K", EPILOGUE)
+def test_linear_epilogue(dev, M, N, K):
+    test_linear_ring(dev, M, N, K, False)
+    test_linear_ring(dev, M, N, K, True)
+
+
+# hidden, intermediate, row counts: the += GEMMs (o_proj, K = 2048, and down) take
+# every fragment-major form, 8 slices at 1024 columns, 4 at 2048
+ALIKE = [(1024, 576, (70, 200, 300, 600, 800, 1100)), (2048, 1088, (70, 200, 300, 400, 520, 600, 700))]
+
+
+@pytest.mark.parametrize("hidden,inter,rows", ALIKE)
+def test_prefill_rows_alike(dev, orc, hidden, inter, rows):
+    """The fewest rows against the oracle; more rows (other forms) give the first
+    ones the same bits."""
+    from qwenasr_amd.model import Decoder
+    from qwenasr_amd.synth import SynthDecoder
+    cfg = dict(n_layers=2, hidden=hidden, n_heads=16, n_kv_heads=8, head_dim=128, intermediate=inter, vocab=1000,
+               eps=1e-6, theta=1e6)
+    w = SynthDecoder(cfg, seed=78)
+    d = Decoder(dev, w, max_seq=1280)
+    emb = rng(hidden).normal(0, 0.02, (rows[-1], hidden)).astype(np.float32)
+    logits, kv = {}, {}
+    for n in rows:
+        print(f"prefill rows alike hidden={hidden} rows={n}", flush=True)
+        d.kv_len = 0
+        logits[n] = d.prefill_logits(emb[:n])
+        kv[n] = d.kv_rows_download(0, n)
+    d.close()
+    n0 = rows[0]
+    cpu = orc.OracleDecoder(w, max_seq=256)
+    want = cpu.prefill_logits(emb[:n0])
+    kc, vc = cpu.kv()
+    cpu.close()
+    for got, ref in ((kv[n0][0], kc[:, :, :n0]), (kv[n0][1], vc[:, :, :n0])):
+        assert np.linalg.norm(got - ref) <= 1e-5 * np.linalg.norm(ref)
+    assert np.linalg.norm(logits[n0] - want) <= 2e-4 * np.linalg.norm(want)
+    for a, b in zip(rows, rows[1:]):
+        assert (logits[b][:a] == logits[a]).all(), (a, b)
+        assert all((kv[b][i][:, :, :a] == kv[a][i]).all() for i in range(2)), (a, b)
+
+
+# conv_hidden, whole chunks: conv2 (800 rows a chunk, conv_hidden columns) takes every
+# convolution form
+CONV = [(96, 1), (96, 2), (96, 4), (96, 6), (96, 11), (480, 3)]
+
+
+@pytest.mark.parametrize("conv_hidden,chunks", CONV)
+def test_conv_forms(dev, orc, conv_hidden, chunks):
+    from qwenasr_amd.model import Encoder
+    from qwenasr_amd.synth import SynthEncoder
+    cfg = dict(d_model=64, n_layers=1, n_heads=1, head_dim=64, ffn_dim=128, output_dim=128, chunk_size=100,
+               n_window_infer=800, conv_hidden=conv_hidden)
+    print(f"conv forms conv_hidden={conv_hidden} chunks={chunks}", flush=True)
+    w = SynthEncoder(cfg, seed=60 + conv_hidden)
+    enc, ore = Encoder(dev, w), orc.OracleEncoder(w)
+    mel = rng(chunks).normal(0, 0.5, (128, 100 * chunks + 37)).astype(np.float32)
+    got, want = enc.forward(mel), ore.forward(mel)
+    enc.close()
+    ore.close()
+    # f32-class sums of up to 4320 terms through four convolutions and a layer; measured 2e-7
+    assert got.shape == want.shape
+    assert (np.linalg.norm(got - want, axis=1) <= 1e-5 * np.linalg.norm(want, axis=1).max()).all()
