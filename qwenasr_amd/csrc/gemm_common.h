@@ -12,11 +12,21 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 // lds + 16 l.  Written as inline assembly, with the waits below, because the
 // compiler otherwise treats every LDS read as possibly aliasing any load in
 // flight and waits for all of them (vmcnt(0)) before it, which would drain
-// the ring every K-step.  The compiler does not see these loads: the kernels
-// issue no other vector-memory load until their final vmcnt(0), and make no
-// other use of M0 (the generated code was checked for both).  The s_nop is
-// the wait state GFX9 asks for between a scalar write of M0 and an LDS load
-// that reads it.
+// the stages every step.  The compiler does not see these loads.  Vector-memory
+// loads complete in the order in which a wave issued them, so
+//   - the compiler's own waits, which count only the loads it sees, are at
+//     least as strict as they need to be: a hidden load that is younger than
+//     the one waited for makes vmcnt(n) wait for more, never for less;
+//   - wait_vmcnt<N> here is right where at least N loads of the wave are younger
+//     than the ones it waits for.  k_gemm_lds and k_gemm_ring: the loads of the
+//     NS - 2 stages behind (their other loads come before the first stage or
+//     after the last wait).  k_gemm_ks: N = 0.  k_attn_mfma and k_attn_bf3: the
+//     L loads of the next K tile or of the V tile; q is loaded behind the first
+//     two tiles and waited for ahead of the loop.
+// The compiler makes no use of M0 in the kernels of the files that include this
+// header (every mention of it in their generated code is one of these lines).
+// The s_nop is the wait state GFX9 asks for between a scalar write of M0 and
+// an LDS load that reads it.
 __device__ __forceinline__ void lds_dma16(const void *g, const void *lds) {
     const uint32_t la = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)lds;
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(la) : "memory");

@@ -1,6 +1,6 @@
 """The implicit-im2col GEMM of the encoder's channels-last conv stem finds the
 kernel tap of each 32-wide K-step by reciprocal products in float32
-(csrc/k_gemm.hip, A_CONV): t = int((k0 + 16) * (1 / C)), then
+(csrc/k_gemm_ks.hip, A_CONV): t = int((k0 + 16) * (1 / C)), then
 ky = int((t + 0.5) * (1 / kw)).  They must equal the integer quotients for
 every K-step the kernel runs; this checks them, with the kernel's float32
 rounding (no fused multiply-add), for every width C = 32 ... 4096 that is a
