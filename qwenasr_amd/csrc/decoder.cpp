@@ -489,7 +489,7 @@ static int run_step_graph(qasr_decoder *d, int64_t cap, int n) {
             d->step_pos += 1;
         }
         d->step_pos = pos0;
-        d->step_report = true;
+        d->step_report = false;
         hipError_t e = hipStreamEndCapture(d->h->stream, &g);
         if (rc != QASR_OK) {
             if (g) (void)hipGraphDestroy(g);
@@ -545,13 +545,18 @@ extern "C" int qasr_hip_decoder_forward(qasr_decoder *d, const float *embed, int
     if (!embed && (token_in < 0 || token_in >= d->c.vocab))
         return qasr_fail(QASR_ERR_INVALID, "decoder_forward: token id out of range");
     TRY(set_state(d, token_in));
-    if (embed) {
+    if (embed)
         HIPCHK(hipMemcpyAsync(d->x, embed, sizeof(float) * d->c.hidden, hipMemcpyHostToDevice, d->h->stream));
-        TRY(decoder_enqueue_step(d, false));
+    d->step_report = true;
+    int rc;
+    if (embed) {
+        rc = decoder_enqueue_step(d, false);
         d->step_pos += 1;
     } else {
-        TRY(decoder_run_embed_step(d));
+        rc = decoder_run_embed_step(d);
     }
+    d->step_report = false;
+    TRY(rc);
     // the step reported its token, fault flag and logit to pinned host memory:
     // one wait, no copies
     HIPCHK(hipStreamSynchronize(d->h->stream));

@@ -52,10 +52,11 @@ struct qasr_decoder {
     // partition is sized for the bucket); keyed by the bucket's capacity
     std::map<int64_t, hipGraphExec_t> graphs;
     int64_t step_pos = 0;                       // position of the next step to enqueue
-    // pinned: {token, position, fault, logit bits} of the last single step,
-    // written by its argmax merge (null inside a captured run of several)
+    // pinned: {token, position, fault, logit bits} of decoder_forward's last
+    // step, written by its argmax merge (steps captured one by one report
+    // too: their graph is decoder_forward's; others do not, 0.4 us each)
     int32_t *host_rep = nullptr;
-    bool step_report = true;                    // steps enqueued now report to host_rep
+    bool step_report = false;                   // steps enqueued now report to host_rep
     bool rep_valid = false;                     // host_rep is the decoder's last step (read after a synchronisation)
     PrefillBufs pf;
     DevBuf head_out;                            // prefill_logits / prefill_argmax outputs, kept between calls
