@@ -208,11 +208,10 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(GemmArgs g) {
 // the wait count is the same in every iteration.  Requires K % 64 == 0 and
 // 16-byte aligned rows.
 //
-// VEC (N a multiple of 4, 16-byte aligned C rows, K >= 512): the columns are the
-// MFMA's rows, so a lane ends with 4 consecutive columns and stores 16 bytes (the
-// same bits).  Other N keep a column per lane: 16
-// consecutive floats per store, where 4 scalar stores of the other layout would
-// be 4 rows apart each (424 x 82070 x 1024 102 -> 144 us).
+// VEC (N a multiple of 4, 16-byte aligned C rows): the columns are the MFMA's
+// rows, so a lane ends with 4 consecutive columns and stores 16 bytes; else a
+// column per lane (16 consecutive floats per store).  The same bits; the
+// dispatch below says where which is faster.
 //
 // KP > 1 splits the K loop inside the block: 4 KP waves in KP groups of 4,
 // group p taking the K-steps p, p + KP, ... through a ring of its own; at the
@@ -238,7 +237,7 @@ __global__ __launch_bounds__(256 * KP, BM * BN > 64 * 64 ? 2 : 1) void k_gemm_ld
     constexpr int LA = BM / 32, LB = BN / 64;                        // one-KiB loads per wave per stage
     // wave tiling: int8 B, which needs converting, is owned by one wave per
     // fragment (BN/4-column strips), so no fragment is converted twice.
-    // (Measured and rejected for the LM head at M = 375: 2 x 2 waves of
+    // (Measured and rejected for the LM head at M = 375, in loops: 2 x 2 waves of
     // (BM/2) x (BN/2), which halve the A reads from LDS but widen every B
     // fragment in two waves: 143 -> 160 us with 128 x 128 tiles, 157-167 with
     // 192 x 128 and 128 x 256; 8 waves on 128 x 256 tiles 156-162.)
@@ -290,19 +289,20 @@ __global__ __launch_bounds__(256 * KP, BM * BN > 64 * 64 ? 2 : 1) void k_gemm_ld
 
     // The column scales do not depend on the products: loaded before the
     // ring's first stage, so that no load is left after the K loop.  Being
-    // older than every ring load, they are complete by the first wait.
+    // older than every ring load, they are complete by the first wait.  (By every
+    // group, though group 0 alone uses them: under a test of the group the
+    // pointer's argument load falls behind the others, a round trip more before
+    // the first stage: 33 x 10001 x 1024 in 64 x 64 tiles 7.7 -> 7.3 us.)
     const int fr = lane & 15, fg = lane >> 4;
     f32x4 pre_s[WC];
-    if (grp == 0) {
-        const bool sv = ((uintptr_t)g.scale & 15) == 0;
+    const bool sv = ((uintptr_t)g.scale & 15) == 0;
 #pragma unroll
-        for (int j = 0; j < WC; j++) {
-            if constexpr (VEC) {
-                pre_s[j] = gemm_load4(g.scale, min(n0 + nw + j * 16 + 4 * fg, N - 1), N, sv);
-            } else {
-                const float x = g.scale[min(n0 + nw + j * 16 + fr, N - 1)];
-                pre_s[j] = f32x4{x, x, x, x};
-            }
+    for (int j = 0; j < WC; j++) {
+        if constexpr (VEC) {
+            pre_s[j] = gemm_load4(g.scale, min(n0 + nw + j * 16 + 4 * fg, N - 1), N, sv);
+        } else {
+            const float x = g.scale[min(n0 + nw + j * 16 + fr, N - 1)];
+            pre_s[j] = f32x4{x, x, x, x};
         }
     }
 
@@ -313,7 +313,7 @@ __global__ __launch_bounds__(256 * KP, BM * BN > 64 * 64 ? 2 : 1) void k_gemm_ld
         __syncthreads();                      // ... and every wave's; stage kt - 1 is free
         issue((kt + NS - 1) % NS, kt + NS - 1);
         const char *st = smem[kt % NS];
-        if (BN == 128) __builtin_amdgcn_iglp_opt(1);   // LDS reads spread between the MFMAs (LM head 143 -> 141 us)
+        if (BN == 128) __builtin_amdgcn_iglp_opt(1);   // LDS reads spread between the MFMAs
 #pragma unroll
         for (int s = 0; s < BK / 32; s++) {
             bf16x8 bfrag[WC];
@@ -477,11 +477,9 @@ static hipError_t go_gemm(const GemmArgs &g, int epi, hipStream_t st) {
 // count of rounds (several blocks share a CU).  The figures are fits, in 0.1 us
 // at K = 1024, to a sweep over M = 16 ... 404 and N = 4096 ... 151936; one (64 x
 // 128) is raised for K = 2048 and 3072, where two 64 x 64 tiles are faster.  K <
-// 512, where a tile's fixed part weighs more, has figures of its own and stores a
-// column per lane (256 x 20000 x 192 11.3 -> 9.1 us, 375 x 60000 x 256 32.2 ->
-// 28.3 by both).  A third row for K from 1536 on was fitted too: 0.5%
-// faster on average over 262 shapes, the LM head at M = 375 3% slower.  us per
-// launch with 64 x 64 tiles below 2048 of them and 128 x 128 beyond, then by
+// 512, where a tile's fixed part weighs more, has figures of its own (256 x 20000
+// x 192 11.2 -> 9.2 us).  Rows fitted to more shapes gained 0.5% on those and lost
+// 0.3% (up to 15%) on 172 others; they were not taken.  us per launch with 64 x 64 tiles below 2048 of them and 128 x 128 beyond, then by
 // this rule: M = 16, N = 60001 17.2 -> 14.0, N = 151936 42.2 -> 27.0; M = 64, N
 // = 151936 46.6 -> 37.0; M = 90, N = 60001 36.6 -> 27.6; M = 140, N = 151936
 // 88.6 -> 65.4; M = 375, N = 20000 32.2 -> 24.0; M = 404, N = 151936 182 -> 170.
@@ -491,13 +489,27 @@ static hipError_t go_gemm(const GemmArgs &g, int epi, hipStream_t st) {
 // against 155); each block walking every M tile of its strip (205); non-temporal
 // stores of C (143 -> 147); the activations split into three int8 planes on the
 // int8 MFMA (273-282: three bytes per activation through the ring).
+//
+// 16-byte stores (VEC), on buffers that are not in the cache: 64 x 64 tiles always
+// (375 x 4096 x 1024 10.5 -> 10.25 us), 32 x 64 in more than one round of tiles
+// (90 x 6144 7.7 -> 7.5; in one round 5.8 -> 6.0), 128 columns in one round (375 x
+// 10000 16.3 -> 15.6; in more, where a tile's stores run beside the next tile's
+// K loop, the longer runs of single rows are better: LM head at M = 375 159 ->
+// 152, 190 x 60000 39.9 -> 37.8).
 struct W8Form { int bm, bn, one, more; };
 
-template <bool VEC>
+template <int NS, int BM, int BN, int KP>
+static void go_w8(const GemmArgs &g, bool vec, hipStream_t st) {
+    const dim3 grid((g.N + BN - 1) / BN, (g.M + BM - 1) / BM);
+    if (vec) hipLaunchKernelGGL((k_gemm_lds<NS, BM, BN, KP, true>), grid, dim3(256 * KP), 0, st, g);
+    else hipLaunchKernelGGL((k_gemm_lds<NS, BM, BN, KP, false>), grid, dim3(256 * KP), 0, st, g);
+}
+
 static hipError_t go_gemm_lds(const GemmArgs &g, hipStream_t st) {
+    const bool vec = g.N % 4 == 0 && g.ldc % 4 == 0 && (uintptr_t)g.C % 16 == 0;
     const int64_t small_blocks = (int64_t)((g.N + 63) / 64) * ((g.M + 63) / 64);
     if (small_blocks < 2048 && g.K / 64 >= 16 && (g.N + 63) / 64 <= 32) {
-        hipLaunchKernelGGL((k_gemm_lds<3, 64, 64, 4, VEC>), dim3((g.N + 63) / 64, (g.M + 63) / 64), dim3(1024), 0, st, g);
+        go_w8<3, 64, 64, 4>(g, vec, st);
         return hipGetLastError();
     }
     static const W8Form longk[] = {{32, 64, 64, 26}, {64, 64, 80, 37}, {64, 128, 125, 68},
@@ -514,14 +526,15 @@ static hipError_t go_gemm_lds(const GemmArgs &g, hipStream_t st) {
         const int64_t c = 512 * (int64_t)f[i].one + (rounds > 1 ? f[i].more * (tiles + 256 * rounds - 512) : 0);
         if (c < best_cost) { best_cost = c; best = i; }
     }
-    const dim3 grid((g.N + f[best].bn - 1) / f[best].bn, (g.M + f[best].bm - 1) / f[best].bm);
+    const int64_t tiles = (int64_t)((g.M + f[best].bm - 1) / f[best].bm) * ((g.N + f[best].bn - 1) / f[best].bn);
+    const bool one_round = tiles <= 256;
     switch (best) {
-        case 0: hipLaunchKernelGGL((k_gemm_lds<4, 32, 64, 1, VEC>), grid, dim3(256), 0, st, g); break;
-        case 1: hipLaunchKernelGGL((k_gemm_lds<4, 64, 64, 1, VEC>), grid, dim3(256), 0, st, g); break;
-        case 2: hipLaunchKernelGGL((k_gemm_lds<2, 64, 128, 1, VEC>), grid, dim3(256), 0, st, g); break;
-        case 3: hipLaunchKernelGGL((k_gemm_lds<2, 96, 128, 1, VEC>), grid, dim3(256), 0, st, g); break;
-        case 4: hipLaunchKernelGGL((k_gemm_lds<2, 128, 128, 1, VEC>), grid, dim3(256), 0, st, g); break;
-        default: hipLaunchKernelGGL((k_gemm_lds<2, 160, 128, 1, VEC>), grid, dim3(256), 0, st, g); break;
+        case 0: go_w8<4, 32, 64, 1>(g, vec && !one_round, st); break;
+        case 1: go_w8<4, 64, 64, 1>(g, vec, st); break;
+        case 2: go_w8<2, 64, 128, 1>(g, vec && one_round, st); break;
+        case 3: go_w8<2, 96, 128, 1>(g, vec && one_round, st); break;
+        case 4: go_w8<2, 128, 128, 1>(g, vec && one_round, st); break;
+        default: go_w8<2, 160, 128, 1>(g, vec && one_round, st); break;
     }
     return hipGetLastError();
 }
@@ -551,8 +564,7 @@ hipError_t launch_gemm(const GemmArgs &g0, int asrc, int bsrc, int epi, hipStrea
         const bool ring = epi == EPI_SCALE && !g.bias && g.K % 64 == 0 && (g.lda * 2) % 16 == 0 && g.ldb % 16 == 0 &&
                           (uintptr_t)g.A % 16 == 0 && (uintptr_t)g.B % 16 == 0;
         if (!ring) return go_gemm<A_BF16, B_I8>(g, epi, st);
-        const bool vec = g.K >= 512 && g.N % 4 == 0 && g.ldc % 4 == 0 && (uintptr_t)g.C % 16 == 0;
-        return vec ? go_gemm_lds<true>(g, st) : go_gemm_lds<false>(g, st);
+        return go_gemm_lds(g, st);
     }
     if (asrc == A_BF16 && bsrc == B_BF16) return go_gemm<A_BF16, B_BF16>(g, epi, st);
     return hipErrorInvalidValue;

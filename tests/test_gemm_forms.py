@@ -26,9 +26,9 @@ def rows_of(text, width):
 
 
 def w8_form(M, N, K):
-    """go_gemm_lds' choice: (rows, columns) of the tile, or "K groups"."""
+    """go_gemm_lds' choice: (rows, columns) of the tile, or "K groups"; 16-byte stores."""
     if up(N, 64) * up(M, 64) < 2048 and K // 64 >= 16 and up(N, 64) <= 32:
-        return "K groups"
+        return "K groups", N % 4 == 0
     src = source("k_gemm.hip")
     name = "shortk" if K < 512 else "longk"
     forms = rows_of(re.search(r"W8Form " + name + r"\[\] = \{(.*?)\};", src, re.S).group(1), 4)
@@ -38,20 +38,23 @@ def w8_form(M, N, K):
         tiles = up(M, f[0]) * up(N, f[1])
         rounds = up(tiles, 256)
         return 512 * f[2] + (f[3] * (tiles + 256 * rounds - 512) if rounds > 1 else 0)
-    return min(forms, key=cost)[:2]
+    f = min(forms, key=cost)[:2]
+    one_round = up(M, f[0]) * up(N, f[1]) <= 256
+    return f, N % 4 == 0 and (f == (64, 64) or one_round == (f[1] == 128))
 
 
 def test_w8_shapes_reach_every_form():
     from test_gpu_w8_forms import EDGES
     seen = {}
     for M, N, K in EDGES:
-        f = w8_form(M, N, K)
-        vec = K >= 512 and N % 4 == 0
+        f, vec = w8_form(M, N, K)
         bm, bn = (64, 64) if f == "K groups" else f
         assert M % bm and N % bn, (M, N, f)          # partial rows and columns
-        seen.setdefault((f, K < 512), set()).add(vec)
+        seen.setdefault(f, set()).add((K < 512, vec))
     tiles = [(32, 64), (64, 64), (64, 128), (96, 128), (128, 128), (160, 128)]
-    assert seen == {**{(t, False): {False, True} for t in tiles + ["K groups"]}, **{(t, True): {False} for t in tiles}}
+    for f in tiles + ["K groups"]:
+        assert {v for _, v in seen[f]} == {False, True}, f
+        assert {k for k, _ in seen[f]} == ({False} if f == "K groups" else {False, True}), f
 
 
 def ks_tables():

@@ -36,11 +36,11 @@ def test_w8_forms(dev, M, N, K):
     assert (y1.numpy()[0] == got[M - 1]).all()
 
 
-# Every form with rows and columns that are no multiple of its tile, with vector (N
-# % 4 == 0 from K = 512 on) and scalar stores, at short and long K: 32 x 64, 64 x 64,
-# 64 x 128, 96 x 128, 128 x 128, 160 x 128, and the K groups (test_gemm_forms.py
-# holds the list to the dispatch's rule)
-EDGES = [(45, 3001, 576), (45, 4100, 576), (75, 8001, 512), (75, 8004, 512), (33, 151937, 512), (33, 151932, 512),
+# Every form with rows and columns that are no multiple of its tile, with vector and
+# scalar stores, at short and long K: 32 x 64, 64 x 64, 64 x 128, 96 x 128, 128 x 128,
+# 160 x 128, and the K groups (test_gemm_forms.py holds the list to the dispatch's
+# rule)
+EDGES = [(45, 3001, 576), (45, 4100, 576), (45, 10004, 576), (75, 8001, 512), (75, 8004, 512), (33, 151937, 512), (33, 151932, 512),
          (75, 20001, 576), (90, 20004, 576), (404, 8001, 512), (404, 8004, 512), (130, 20001, 576), (130, 20004, 576),
          (75, 2003, 1024), (75, 2004, 1088), (45, 3001, 64), (33, 20001, 192), (250, 8004, 64), (75, 30001, 128),
          (404, 8001, 64), (130, 20004, 64)]
