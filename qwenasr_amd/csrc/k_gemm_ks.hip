@@ -14,15 +14,20 @@
 // its own (global_load_lds, refilled as soon as its fragments are in
 // registers), fragment-major B straight into registers (1 KiB contiguous
 // loads), no barrier until the S partial tiles are summed in slice order.
-// What bounds it: per 64 x 64 x 32 step the matrix cores need 192 clk of a CU,
-// the vector memory path 192 (12 KiB at 64 B per clk), and data that passes
-// through LDS 1 clk per 64 B written and per 128 B read; B rows through LDS
-// (plain weights) add half to that, which is why the weights are laid out
-// fragment-major.  Before, four waves shared each K-step of a 64 x 64 tile
-// (24 KiB read from LDS per step, a block barrier per step).  us per launch,
-// cold weights, before -> now (fragment-major):
+// What bounds it, by count: per 64 x 64 x 32 step the matrix cores need 192 clk
+// of a CU, the vector memory path 192 (12 KiB at 64 B per clk), and data that
+// passes through LDS 1 clk per 64 B written and per 128 B read; B rows through
+// LDS (plain weights) add half to that, which is why the weights are laid out
+// fragment-major.  By the counters: the convolutions of 30 s the vector
+// instructions (60% of the issue slots: split and row addresses; MFMA units
+// 44% busy, waits for memory 17% of the waves' time); 404 rows no resource (MFMA
+// 12-25%, waits for memory 20-40%: one K chain per wave, one or two blocks per
+// CU); 67 rows the launch, the first load and the reduction.  Before, four
+// waves shared each K-step of a 64 x 64 tile (24 KiB read from LDS per step, a
+// block barrier per step).  us per launch, cold weights, before -> now
+// (fragment-major):
 //   M = 404: 4096 x 1024  19.3 -> 13.7,  1024 x 2048  16 -> 8.5,
-//            6144 x 1024  28.7 -> 20.9,  1024 x 3072  24 -> 11.9
+//            6144 x 1024  28.7 -> 18.4,  1024 x 3072  24 -> 11.9
 //   M = 67:  4096 x 1024  15.1 -> 6.3,   1024 x 2048  17 -> 5.0,
 //            6144 x 1024  17.1 -> 8.0,   1024 x 3072  23 -> 6.1
 //   conv2 of 30 s (24000 x 480 x 4320) 379 -> 307, conv3 175 -> 88,

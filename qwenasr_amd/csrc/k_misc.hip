@@ -905,7 +905,9 @@ __global__ __launch_bounds__(NW * 64) void k_attn_mfma(AttnRowsArgs a) {
 // with the second's.
 //
 // What bounds it: per tile and two heads 96 MFMAs (1536 clk) and about 550
-// other vector operations (the term splits, the softmax).
+// other vector operations (the term splits, the softmax), which fill 56% of the
+// issue slots at 1337 rows (MFMA units 20% busy, 31% of the waves' time at waits).
+// 1337 rows 163 us on f32 MFMA, 103 with a stage per wave, 78 so.
 //
 // Its range is narrower than f32's: an infinite value, or one of 3.396e38 or
 // more (its bf16 rounding is infinite), has no three terms, and exp_neg has the
@@ -1200,7 +1202,7 @@ __global__ __launch_bounds__(512) void k_attn_bf3(AttnRowsArgs a) {
 
 // Both query heads of a KV head in one block (K and V terms formed once for the
 // two) where that leaves enough blocks: us with one / two heads per block, 672
-// blocks of two (1337 rows) 98.6 / 89.8, 208 (404 rows) 18.1 / 22.9, 40 (67
+// blocks of two (1337 rows) 98.6 / 77, 208 (404 rows) 18.1 / 22.9, 40 (67
 // rows after 337) 13.6 / 21.8.
 static int attn_heads_per_block(int n_kv_heads, int64_t row_blocks) { return n_kv_heads * row_blocks >= 384 ? 2 : 1; }
 

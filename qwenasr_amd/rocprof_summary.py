@@ -3,6 +3,7 @@
     python -m qwenasr_amd.rocprof_summary <dir>/run_kernel_trace.csv [min_batch]
     python -m qwenasr_amd.rocprof_summary --pmc <dir>/run_counter_collection.csv <calib MiB>
     python -m qwenasr_amd.rocprof_summary --traffic <fetch csv> <write csv> <calib MiB> > profiles/hbm_traffic.txt
+    python -m qwenasr_amd.rocprof_summary --counters <dir>/run_kernel_trace.csv <counter csv> ...
     python -m qwenasr_amd.rocprof_summary --mfma-config1 <MfmaUtil csv> <MOPS csv> [reps [<FETCH csv> <WRITE csv> <calib MiB>]]
 
 The second form averages each kernel's counter values (``--pmc FETCH_SIZE`` or
@@ -10,6 +11,11 @@ The second form averages each kernel's counter values (``--pmc FETCH_SIZE`` or
 the library's copy kernel (``k_copy16``) moving a known number of MiB
 (bench.py ``--copy-calib-mb``): bytes per dispatch = value * calib_bytes /
 copy_value.
+
+The --counters form lists every (kernel, blocks) of the counter files with the
+median of its durations in the trace and of each counter (FETCH_SIZE and
+WRITE_SIZE in MB, scaled by the 64 MiB copy if the run made one; SQ_ACTIVE_* and
+SQ_WAIT_* as shares of SQ_WAVE_CYCLES, the bank conflicts of SQ_LDS_IDX_ACTIVE).
 
 Prints a markdown table of every kernel's calls and average / min / max
 duration, and splits the launches of each kernel into those that ran in a
@@ -19,6 +25,7 @@ real decode steps, prefill, encoder, packing).
 """
 import csv
 import hashlib
+import math
 import os
 import re
 import statistics as st
@@ -192,8 +199,53 @@ def mfma_config1(util_csv, mops_csv, reps=3, fetch_csv=None, write_csv=None, cal
     return "\n".join(out)
 
 
+def counters(trace_csv, counter_csvs, calib_mib=64.0):
+    """One row per (kernel, blocks): launches, median us and the counters' medians."""
+    def short(r):
+        return r["Kernel_Name"].split("(")[0].replace("void ", "").replace("qasr::", "")
+    us, vals, names = defaultdict(list), defaultdict(lambda: defaultdict(list)), []
+    for r in csv.DictReader(open(trace_csv)):
+        grid, wg = (math.prod(int(r[f"{k}_{d}"]) for d in "XYZ") for k in ("Grid_Size", "Workgroup_Size"))
+        us[short(r), grid // wg].append((int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3)
+    for path in counter_csvs:
+        per = defaultdict(float)                      # summed over the csv's per-dimension rows
+        for r in csv.DictReader(open(path)):
+            per[int(r["Dispatch_Id"]), short(r), int(r["Grid_Size"]) // int(r["Workgroup_Size"]),
+                r["Counter_Name"]] += float(r["Counter_Value"])
+        for (_, k, b, c), v in per.items():
+            vals[k, b][c].append(v)
+            if c not in names:
+                names.append(c)
+    med = {k: {c: st.median(v) for c, v in d.items()} for k, d in vals.items()}
+    for c in ("FETCH_SIZE", "WRITE_SIZE"):
+        ref = [d[c] for (k, _), d in med.items() if k == "k_copy16" and c in d]
+        scale = calib_mib * 1024 / max(ref) if ref else 1.0
+        for d in med.values():
+            if c in d:
+                d[c] *= scale * 1024 / 1e6
+    shares = {"SQ_LDS_BANK_CONFLICT": "SQ_LDS_IDX_ACTIVE"}
+    shares.update({c: "SQ_WAVE_CYCLES" for c in names if c.startswith(("SQ_ACTIVE_", "SQ_WAIT_"))})
+    show = [c for c in names if c not in shares.values()]
+
+    def cell(d, c):
+        if c not in d:
+            return ""
+        if c in shares:
+            return f"{100 * d[c] / d[shares[c]]:.0f}%" if d.get(shares[c]) else ""
+        return f"{d[c]:.3g}"
+    out = ["| kernel | blocks | launches | us | " + " | ".join(c.replace("SQ_", "") for c in show) + " |",
+           "|---|" + "---:|" * (3 + len(show))]
+    for key, d in sorted(med.items(), key=lambda e: (e[0][0].split("<")[0], -st.median(us.get(e[0], [0])))):
+        if key in us and key[0] != "k_copy16":
+            out.append(f"| `{key[0]}` | {key[1]} | {len(us[key])} | {st.median(us[key]):.1f} | " +
+                       " | ".join(cell(d, c) for c in show) + " |")
+    return "\n".join(out)
+
+
 if __name__ == "__main__":
-    if sys.argv[1] == "--mfma-config1":
+    if sys.argv[1] == "--counters":
+        print(counters(sys.argv[2], sys.argv[3:]))
+    elif sys.argv[1] == "--mfma-config1":
         a = sys.argv
         print(mfma_config1(a[2], a[3], int(a[4]) if len(a) > 4 else 3, *(a[5:7] if len(a) > 7 else ()),
                            *((float(a[7]),) if len(a) > 7 else ())))
