@@ -917,7 +917,9 @@ __global__ __launch_bounds__(NW * 64) void k_attn_mfma(AttnRowsArgs a) {
 // again in plain f32 by the wave that found it (only that row; the others keep
 // their bits).  What this does not see: a q or k value below 2^-109 against one
 // beyond 2^100, and weights below 2^-126 of the largest, which count as 0.
-// The check costs 0.2 us a call (16 rows 6.05 -> 6.25).
+// The check costs 0.2 us a call (16 rows 6.05 -> 6.25); 1337 rows all formed again
+// take 1.9 ms.  (A block's rows formed again together on f32 MFMA, behind a
+// barrier for every block, cost 0.3 us a call.)
 // ---------------------------------------------------------------------------
 // two pairs of f32 -> (hi, mid, lo), two packed dwords each
 __device__ __forceinline__ void split3_4(float x0, float x1, float x2, float x3, uint32_t (&hi)[2], uint32_t (&mi)[2],
